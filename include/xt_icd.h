@@ -122,10 +122,15 @@ enum {
   XT_OPT_BH_QUAD_COEF = 18,  /* BH_QUAD_COEF of the reference build: the beam-hardening
                                 quadratic coefficient of the counts read with sinobin 3
                                 (default 0) */
-  XT_OPT_LINE_GROUP = 19     /* lines a voxel-update workgroup takes at once.  Only 1 is
+  XT_OPT_LINE_GROUP = 19,    /* lines a voxel-update workgroup takes at once.  Only 1 is
                                 accepted in this build: groups of 2 (1 x 2 tiles) and 4
                                 (2 x 2 tiles), updated in turn and writing the error
                                 sinogram once per group, are switched off (default 1) */
+  XT_OPT_PASS = 20           /* how a voxel-update pass runs: 0: automatic; 1: one workgroup per
+                                line in flight; 2: in batches of the lines in flight that read
+                                the same error sinogram, streamed through LDS, wherever the
+                                A-column table and slices of one detector row allow it
+                                (default 0: batches from 16 lines in flight on) */
 };
 int xt_set_option(int option, double value);
 double xt_get_option(int option);

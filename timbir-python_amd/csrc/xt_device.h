@@ -472,16 +472,61 @@ __global__ void __launch_bounds__(256) k_fbp_backproject(XtGeom g, const float *
 }
 
 // ---------------------------------------------------------------------------
+// x^y for x > 0 in FP64, rounded once: log(x) from the series of atanh on
+// [sqrt(1/2), sqrt(2)] (7 terms, 2^-38), exp from its Taylor series (9 terms, 2^-37).
+// FP64 runs at the FP32 vector rate on gfx950: about 45 instructions against 230 of
+// the library's powf, and closer to the exact value (within half an ulp against one).
+__device__ __forceinline__ float xt_powpos(float x, float y) {
+  const double X = (double)x;
+  double m = __builtin_amdgcn_frexp_mant(X);
+  int e = __builtin_amdgcn_frexp_exp(X);
+  const bool low = m < 0.70710678118654752440;
+  m = low ? m + m : m;
+  e = low ? e - 1 : e;
+  const double f = m - 1.0, den = m + 1.0;
+  double q = __builtin_amdgcn_rcp(den);
+  q = __builtin_fma(__builtin_fma(-den, q, 1.0), q, q);
+  const double s = f * q, s2 = s * s;
+  double l = __builtin_fma(s2, 1.0 / 13.0, 1.0 / 11.0);
+  l = __builtin_fma(s2, l, 1.0 / 9.0);
+  l = __builtin_fma(s2, l, 1.0 / 7.0);
+  l = __builtin_fma(s2, l, 1.0 / 5.0);
+  l = __builtin_fma(s2, l, 1.0 / 3.0);
+  l = __builtin_fma(s2, l, 1.0);
+  const double t = (double)y * __builtin_fma(s * l, 2.8853900817779268147, (double)e);
+  const double n = __builtin_rint(t), r = (t - n) * 0.69314718055994530942;
+  double v = __builtin_fma(r, 1.0 / 362880.0, 1.0 / 40320.0);
+  v = __builtin_fma(r, v, 1.0 / 5040.0);
+  v = __builtin_fma(r, v, 1.0 / 720.0);
+  v = __builtin_fma(r, v, 1.0 / 120.0);
+  v = __builtin_fma(r, v, 1.0 / 24.0);
+  v = __builtin_fma(r, v, 1.0 / 6.0);
+  v = __builtin_fma(r, v, 0.5);
+  v = __builtin_fma(r, v, 1.0);
+  v = __builtin_fma(r, v, 1.0);
+  return (float)__builtin_ldexp(v, (int)n);
+}
+
 // qGGMRF surrogate weight b' = b * rho'(delta)/delta (F/XT_ICD_update.c:89-125,
 // 141-168), float.
 __device__ __forceinline__ float xt_qggmrf_ratio(float delta, float p, float c, float sq,
                                                  float sqp) {
   if (delta == 0.f) return 2.0f / (sq * c);
   float ad = fabsf(delta);
-  float t1 = powf(ad, 2.0f - p) / sqp;
+  float t1 = xt_powpos(ad, 2.0f - p) / sqp;
   float t3 = c + t1;
   // rho'(delta)/delta = |delta|^(q-2)/(t3*sq) * (q - (q-p)*t1/t3), q = 2
   return (1.0f / (t3 * sq)) * (2.0f - ((2.0f - p) * t1) / t3);
+}
+
+// The same for q = 2 with its two fractions over one denominator: 2 - (2 - p) t1 / t3 =
+// (2 c + p t1) / t3.
+__device__ __forceinline__ float xt_qggmrf_ratio2(float delta, float p, float c, float sq,
+                                                  float sqp) {
+  if (delta == 0.f) return 2.0f / (sq * c);
+  const float t1 = xt_powpos(fabsf(delta), 2.0f - p) / sqp;
+  const float t3 = c + t1;
+  return (2.0f * c + p * t1) / (t3 * sq * t3);
 }
 
 // Per-launch work description of the voxel-update kernel.
@@ -527,10 +572,6 @@ struct XtIcdBuffers {
                              // graph of one iteration replays for every iteration)
   const uint8_t *vmask;      // [N_time][N_y][N_x][N_z] voxels to update (edge-only
                              // updates), or null: every voxel of a listed line
-  const int *groups;         // line groups of the homogeneous passes: [n_groups][gl]
-                             // member lines (-1: none), adjacent lines of one tile
-  int n_groups;
-  int gl;                    // lines per group (1: the single-line kernel)
 };
 
 // ---------------------------------------------------------------------------
@@ -1066,438 +1107,507 @@ __device__ __forceinline__ void icd_lines_body(const XtGeom &g, const XtIcdBuffe
   }
 }
 
-// ---------------------------------------------------------------------------
-// Voxel-line updates in groups of GL lines (homogeneous passes: the lines of a
-// 1 x 2 or 2 x 2 tile of the image, groups taken in a random order; NHICD and
-// listed lines: GL consecutive entries of the list), with the A columns read
-// from the table.  A group's lines are updated one after another exactly as
-// single lines are (same neighbourhood, theta sums and surrogate), except that
-// the error sinogram is written once per group: line l reads e and subtracts,
-// entry by entry, the changes A_m * delta_m of the group's earlier lines m < l
-// -- the value e would hold had they been applied -- and after the last line
-// one atomic per entry of the union of the group's columns applies the sum of
-// all their changes.  Adjacent lines' columns share most bins, so a 2 x 2
-// group issues about half the atomics of four single lines.  Columns of one
-// view that do not fit the union window of SPAN bins get atomics of their own,
-// so any grouping is exact.  Needs slices of one detector row (zo == 1).
-template <int ZL, bool PACK, int NT, int GL>
-__device__ __forceinline__ void icd_groups_body(const XtGeom &g, const XtIcdBuffers &B,
-                                                const XtIcdLaunch &L, const int bx, const int gx,
-                                                const int f) {
-  static_assert(NT == 64 || NT == 256, "workgroup of one or four waves");
-  static_assert(GL == 2 || GL == 4, "groups of two or four lines");
-  constexpr int ZP = PACK ? ZL / 2 : ZL;  // lanes per view group
-  constexpr int G = NT / ZP;              // view groups
-  constexpr int U = 4;                    // views in flight per group and step
-  constexpr int SPAN = 8;                 // bins of a view's union window
-  constexpr uint32_t OOB = 0x80000000u;   // buffer offset that reads 0 / drops the atomic
-  extern __shared__ float4 smem4[];
-  int *vlist_s = (int *)smem4;                                     // [max_views] view index
-  float *red1 = (float *)(vlist_s + g.max_views);                  // [NT]
-  float *red2 = red1 + NT;                                         // [NT]
-  float *xn = red2 + NT;                                           // [11][ZL]
-  float *dxg = xn + 11 * ZL;                                       // [GL][ZL] changes
-  float *th1z = dxg + GL * ZL;                                     // [ZL]
-  float *th2z = th1z + ZL;                                         // [ZL]
-  float *magb = th2z + ZL;                                         // [64]
-  __shared__ int s_cnt_col, s_perf;
-
-  const int tid = threadIdx.x;
-  const int nv = B.proj_num[f];
-  const size_t NYX = (size_t)g.N_y * g.N_x;
-  const int iter = *B.iter;
-  const int blk_sz = g.N_z / g.nb;
-  const int par = (L.mode == 2) ? -1 : ((L.half ^ f) & 1);
-  const int grp = tid / ZP, lz = tid % ZP;
-  int zs = lz;
-  if constexpr (PACK) zs = ((lz / blk_sz) * 2 + par) * blk_sz + lz % blk_sz;
-  auto zblock = [&](int z) {
-    int b = blk_sz > 0 ? z / blk_sz : g.nb - 1;
-    return b >= g.nb ? g.nb - 1 : b;
-  };
-  const bool zs_ok = zs < g.N_z && (par < 0 || (zblock(zs) & 1) == par);
-  for (int p = tid; p < nv; p += NT) vlist_s[p] = B.views[(size_t)f * g.max_views + p];
-
-  // ---- this launch's items: groups of the random order (mode 0); runs of GL
-  // consecutive entries of the workgroup's contiguous share of the NHICD list
-  // (mode 1) or of the line list (modes 2, 3: items bx, bx + gx, ...)
-  int n_items = 0, i0 = 0, istep = 1, r0 = 0, r1 = 0, n_dom = 0;
-  const int *list = B.lines;
-  uint32_t key = 0;
-  if (L.mode == 0) {
-    const int n = B.n_groups;
-    const int per = n / L.K;
-    const int lo = L.sub_iter * per;
-    n_items = (L.sub_iter == L.K - 1) ? n : (L.sub_iter + 1) * per;
-    i0 = lo + bx;
-    istep = gx;
-    n_dom = n;
-    key = xt_order_key(L.seed, iter, f, par);
-  } else if (L.mode == 1) {
-    const int hi = B.nhicd_count[f * 2 + par];
-    list = B.nhicd_list + ((size_t)f * 2 + par) * NYX;
-    key = xt_hash(L.seed ^ 0x5BD1E995u ^ xt_hash((uint32_t)iter * 0xC2B2AE35u ^ (uint32_t)f));
-    r0 = (int)((long long)hi * bx / gx);
-    r1 = (int)((long long)hi * (bx + 1) / gx);
-    n_items = (r1 - r0 + GL - 1) / GL;
-  } else {
-    r1 = B.n_lines;
-    n_items = (r1 + GL - 1) / GL;
-    i0 = bx;
-    istep = gx;
-  }
-  if (tid == 0) {
-    s_cnt_col = 0;
-    s_perf = 0;
-  }
-  float vox_mag = 0.f;
-  double n_upd = 0.0, n_foot = 0.0, n_vis = 0.0;
-  const size_t tbl = (size_t)f * NYX * g.max_views;
-  const uint32_t sino_bytes = (uint32_t)((size_t)g.N_p * g.N_r * g.N_t * sizeof(float));
-  const __amdgpu_buffer_rsrc_t rs_e = __builtin_amdgcn_make_buffer_rsrc(B.e, 0, sino_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_w =
-      __builtin_amdgcn_make_buffer_rsrc((void *)B.w, 0, sino_bytes, 0x00020000);
-  const int bin_bytes = (g.pm ? g.H : g.N_t) * (int)sizeof(float);
-  const int plane = g.pm ? par * g.N_p * g.N_r * g.H : 0;
-  const int row_len = g.pm ? g.H : g.N_t;
-  const uint32_t lane_off = (uint32_t)(g.pm ? lz : zs) * sizeof(float);
-  const float T2 = g.T * g.T, Td = g.T * g.delta, dt = g.delta_t;
-  __syncthreads();
-
-  for (int i = i0; i < n_items; i += istep) {
-    int cl[GL];
-    uint32_t gkey;
-    if (L.mode == 0) {
-      const int gi = xt_permute(i, n_dom, key);
-#pragma unroll
-      for (int m = 0; m < GL; m++) cl[m] = B.groups[(size_t)gi * GL + m];
-      gkey = (uint32_t)gi;
-    } else {
-      const int e0 = r0 + i * GL;
-#pragma unroll
-      for (int m = 0; m < GL; m++) cl[m] = e0 + m < r1 ? list[e0 + m] : -1;
-      gkey = (uint32_t)cl[0];
-    }
-    const int rot = (int)(xt_hash(gkey * 0x27D4EB2Fu ^ key ^ (uint32_t)L.half) %
-                          (uint32_t)(nv > 0 ? nv : 1));
-    for (int q = tid; q < GL * ZL; q += NT) dxg[q] = 0.f;
-
-    for (int l = 0; l < GL; l++) {
-      const int c = cl[l];
-      if (c < 0) continue;  // the same for every thread of the workgroup
-      const int yy = c / g.N_x, xx = c - yy * g.N_x;
-      const bool lane_on =
-          zs_ok && (L.mode != 1 || B.nhicd_blk[((size_t)f * g.nb + zblock(zs)) * NYX + c] != 0);
-      const size_t row_l = tbl + (size_t)c * g.max_views;
-      // ---- neighbourhood (the group's earlier lines are already written back)
-      // and the column's entry count
-      int cnt_local = 0;
-      for (int p = tid; p < nv; p += NT) {
-        const float4 t4 = B.at_vals[row_l + p];
-        cnt_local += (t4.x > 0.f) + (t4.y > 0.f) + (t4.z > 0.f) + (t4.w > 0.f);
-      }
-      for (int q = tid; q < 11 * ZL; q += NT) {
-        const int k = q / ZL, z = q - k * ZL;
-        float val = 0.f;
-        if (z < g.N_z) {
-          if (k < 9) {
-            const int y2 = yy + k / 3 - 1, x2 = xx + k % 3 - 1;
-            if (y2 >= 0 && y2 < g.N_y && x2 >= 0 && x2 < g.N_x)
-              val = __hip_atomic_load(&B.x[((size_t)f * NYX + (size_t)y2 * g.N_x + x2) * g.N_z + z],
-                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          } else {
-            const int f2 = f + (k == 9 ? -1 : 1);
-            if (f2 >= 0 && f2 < g.N_time)
-              val = __hip_atomic_load(&B.x[((size_t)f2 * NYX + c) * g.N_z + z], __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-        xn[q] = val;
-      }
-      if (cnt_local) atomicAdd(&s_cnt_col, cnt_local);
-      __syncthreads();
-
-      // ---- theta pass over e less the group's earlier lines' changes
-      float dprev[GL];
-#pragma unroll
-      for (int m = 0; m < GL; m++) dprev[m] = (m < l && zs < ZL) ? dxg[m * ZL + zs] * dt : 0.f;
-      bool corr = false;
-#pragma unroll
-      for (int m = 0; m < GL; m++) corr |= dprev[m] != 0.f;
-      float th1 = 0.f, th2 = 0.f;
-      if (lane_on) {
-        for (int q0 = grp; q0 < nv; q0 += U * G) {
-          uint32_t off[U];
-          int first[U], pv[U];
-          float av[U][4], ev[U][4], wv[U][4];
-#pragma unroll
-          for (int u = 0; u < U; u++) {
-            const int q = q0 + u * G;
-            int p = q + rot;
-            if (p >= nv) p -= nv;
-            const bool ok = q < nv;
-            pv[u] = ok ? p : -1;
-            const float4 t4 = ok ? B.at_vals[row_l + p] : make_float4(0.f, 0.f, 0.f, 0.f);
-            first[u] = ok ? B.at_first[row_l + p] : 0;
-            av[u][0] = t4.x * dt;
-            av[u][1] = t4.y * dt;
-            av[u][2] = t4.z * dt;
-            av[u][3] = t4.w * dt;
-            off[u] = ok ? (uint32_t)(plane + (vlist_s[p] * g.N_r + first[u]) * row_len) *
-                                  (uint32_t)sizeof(float) + lane_off
-                        : OOB;
-          }
-#pragma unroll
-          for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-              const uint32_t o = av[u][b] > 0.f ? off[u] : OOB;
-              ev[u][b] =
-                  __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_e, o, b * bin_bytes, 0));
-              wv[u][b] =
-                  __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_w, o, b * bin_bytes, 0));
-            }
-          if (corr) {
-            // e -= A_m * delta_m of the earlier lines where their columns meet this one's
-#pragma unroll
-            for (int m = 0; m < GL - 1; m++) {
-              if (m < l && cl[m] >= 0) {
-                const size_t rm = tbl + (size_t)cl[m] * g.max_views;
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                  if (pv[u] >= 0) {
-                    const float4 t4 = B.at_vals[rm + pv[u]];
-                    const int k0 = first[u] - B.at_first[rm + pv[u]];
-                    const float am[4] = {t4.x, t4.y, t4.z, t4.w};
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                      const int k = k0 + b;
-                      float a = 0.f;
-#pragma unroll
-                      for (int kk = 0; kk < 4; kk++) a = (k == kk) ? am[kk] : a;
-                      ev[u][b] -= a * dprev[m];
-                    }
-                  }
-                }
-              }
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-              const float pe = av[u][b], e1 = ev[u][b], w1 = wv[u][b];
-              // generalized Huber weight as in the single-line kernel
-              const float wr = Td * __builtin_amdgcn_sqrtf(w1) * __builtin_amdgcn_rcpf(fabsf(e1));
-              const float ws = (e1 * e1 * w1 < T2) ? w1 : wr;
-              const float pw = pe * ws;
-              th2 += pe * pw;
-              th1 -= e1 * pw;
-            }
-        }
-      }
-      red1[tid] = th1;
-      red2[tid] = th2;
-      __syncthreads();
-      if (tid < ZP) {
-        float t1 = 0.f, t2 = 0.f;
-        for (int q = 0; q < G; q++) {
-          t1 += red1[q * ZP + tid];
-          t2 += red2[q * ZP + tid];
-        }
-        if (zs < ZL) {
-          th1z[zs] = t1;
-          th2z[zs] = t2;
-        }
-      }
-      if (tid < 64) magb[tid] = 0.f;
-      __syncthreads();
-
-      // ---- surrogate update of the active slices, red-black in z (or ascending)
-      float *xcol = xn + 4 * ZL;
-      const int n_steps = L.zorder ? g.N_z : 2;
-      for (int step = 0; step < n_steps; step++) {
-        const int z = tid;
-        bool upd = false;
-        if (z < g.N_z && (L.zorder ? (z == step) : ((z & 1) == step))) {
-          upd = par < 0 || (zblock(z) & 1) == par;
-          if (upd && L.mode == 1) upd = B.nhicd_blk[((size_t)f * g.nb + zblock(z)) * NYX + c] != 0;
-          if (upd && B.vmask) upd = B.vmask[((size_t)f * NYX + c) * g.N_z + z] != 0;
-        }
-        if (upd) {
-          const float V = xcol[z];
-          float nb[27];
-          bool fl[27];
-          bool any_pos = false;
-#pragma unroll
-          for (int dz = -1; dz <= 1; dz++)
-#pragma unroll
-            for (int dy = -1; dy <= 1; dy++)
-#pragma unroll
-              for (int dx = -1; dx <= 1; dx++) {
-                const int ll = ((dz + 1) * 3 + (dy + 1)) * 3 + (dx + 1);
-                const int z2 = z + dz, y2 = yy + dy, x2 = xx + dx;
-                const bool ok = (ll != 13) && z2 >= 0 && z2 < g.N_z && y2 >= 0 && y2 < g.N_y &&
-                                x2 >= 0 && x2 < g.N_x;
-                const float val = ok ? xn[((dy + 1) * 3 + (dx + 1)) * ZL + z2] : 0.f;
-                nb[ll] = val;
-                fl[ll] = ok;
-                any_pos |= ok && (val > 0.f);
-              }
-          const bool tf0 = f > 0, tf1 = f + 1 < g.N_time;
-          const float tn0 = xn[9 * ZL + z], tn1 = xn[10 * ZL + z];
-          any_pos |= (tf0 && tn0 > 0.f) || (tf1 && tn1 > 0.f);
-          const bool skip = (V == 0.f) && (iter > 1) && !any_pos;
-          if (!skip) {
-            float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int ll = 0; ll < 27; ll++) {
-              if (fl[ll]) {
-                const float bq = g.filt[ll] *
-                                 xt_qggmrf_ratio(V - nb[ll], g.MRF_P, g.C_S, g.Sigma_S_Q, g.Sigma_S_Q_P);
-                s1 += bq * nb[ll];
-                s2 += bq;
-              }
-            }
-            if (tf0) {
-              const float bq =
-                  g.tfilt * xt_qggmrf_ratio(V - tn0, g.MRF_P, g.C_T, g.Sigma_T_Q, g.Sigma_T_Q_P);
-              s1 += bq * tn0;
-              s2 += bq;
-            }
-            if (tf1) {
-              const float bq =
-                  g.tfilt * xt_qggmrf_ratio(V - tn1, g.MRF_P, g.C_T, g.Sigma_T_Q, g.Sigma_T_Q_P);
-              s1 += bq * tn1;
-              s2 += bq;
-            }
-            const float T1 = th1z[z], T2z = th2z[z];
-            const float u = (s1 + (T2z * V) - T1) / (s2 + T2z);
-            float nv2 = V + g.alpha * (u - V);
-            if (g.positivity && nv2 <= 0.f) nv2 = 0.f;
-            xcol[z] = nv2;
-            dxg[l * ZL + z] = nv2 - V;
-            atomicAdd(&magb[zblock(z)], fabsf(nv2 - V));
-            vox_mag += fabsf(nv2);
-            atomicAdd(&s_perf, 1);
-          }
-        }
-        __syncthreads();
-      }
-      // ---- write the line back and its update magnitude
-      if (tid < g.N_z)
-        __hip_atomic_store(&B.x[((size_t)f * NYX + c) * g.N_z + tid], xcol[tid], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      if (tid < g.nb) {
-        const size_t mi = ((size_t)f * g.nb + tid) * NYX + c;
-        if ((par < 0 || (tid & 1) == par) && (L.mode != 1 || B.nhicd_blk[mi] != 0))
-          B.mag_blk[mi] = magb[tid];
-        else
-          magb[tid] = B.mag_blk[mi];
-      }
-      __syncthreads();
-      if (tid == 0) {
-        float sm = 0.f;
-        for (int b = 0; b < g.nb; b++) sm += magb[b];
-        B.magsum[(size_t)f * NYX + c] = sm;
-        n_upd += (double)s_perf;
-        n_foot += (double)s_perf * (double)s_cnt_col;
-        n_vis += 1.0;
-        s_cnt_col = 0;
-        s_perf = 0;
-      }
-      // the next line's neighbourhood loads must see this line's values
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-    }
-
-    // ---- e -= sum over the group's lines of A_m * delta_m: per view one atomic
-    // per bin of the window [u0, u0 + SPAN) from the leftmost column, columns
-    // reaching past it on their own
-    float dzm[GL];
-    bool any = false;
-#pragma unroll
-    for (int m = 0; m < GL; m++) {
-      dzm[m] = (zs < ZL && zs_ok) ? dxg[m * ZL + zs] * dt : 0.f;
-      any |= dzm[m] != 0.f;
-    }
-    if (any) {
-      for (int q = grp; q < nv; q += G) {
-        int p = q + rot;
-        if (p >= nv) p -= nv;
-        float am[GL][4];
-        int fm[GL];
-        int u0 = 0x7fffffff;
-#pragma unroll
-        for (int m = 0; m < GL; m++) {
-          float4 t4 = make_float4(0.f, 0.f, 0.f, 0.f);
-          fm[m] = 0;
-          if (cl[m] >= 0) {
-            const size_t rm = tbl + (size_t)cl[m] * g.max_views + p;
-            t4 = B.at_vals[rm];
-            fm[m] = B.at_first[rm];
-            u0 = min(u0, fm[m]);
-          }
-          am[m][0] = t4.x;
-          am[m][1] = t4.y;
-          am[m][2] = t4.z;
-          am[m][3] = t4.w;
-        }
-        const uint32_t vrow = (uint32_t)(plane + vlist_s[p] * g.N_r * row_len);
-        const uint32_t o = (vrow + (uint32_t)(u0 * row_len)) * (uint32_t)sizeof(float) + lane_off;
-        bool out[GL];
-#pragma unroll
-        for (int m = 0; m < GL; m++) out[m] = fm[m] + 4 > u0 + SPAN;
-#pragma unroll
-        for (int b = 0; b < SPAN; b++) {
-          float d = 0.f;
-#pragma unroll
-          for (int m = 0; m < GL; m++) {
-            const int k = u0 + b - fm[m];
-            float a = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) a = (k == kk) ? am[m][kk] : a;
-            d += out[m] ? 0.f : a * dzm[m];
-          }
-          __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(-d, rs_e, d != 0.f ? o : OOB,
-                                                        b * bin_bytes, 0);
-        }
-#pragma unroll
-        for (int m = 0; m < GL; m++) {
-          if (out[m]) {
-            const uint32_t om = (vrow + (uint32_t)(fm[m] * row_len)) * (uint32_t)sizeof(float) + lane_off;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-              const float d = am[m][b] * dzm[m];
-              __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(-d, rs_e, d != 0.f ? om : OOB,
-                                                            b * bin_bytes, 0);
-            }
-          }
-        }
-      }
-    }
-    // the next group's loads must see these atomics
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  if (tid < ZL && L.count_stats && vox_mag != 0.f) atomicAdd(&B.stats[0], (double)vox_mag);
-  if (tid == 0 && n_vis != 0.0) {
-    atomicAdd(&B.stats[1], n_upd);
-    atomicAdd(&B.stats[2], n_foot);
-    atomicAdd(&B.stats[3], n_vis);
-  }
-}
-
-template <int ZL, bool PACK, int NT, int GL>
-__global__ void __launch_bounds__(NT) k_icd_groups(XtGeom g, XtIcdBuffers B, XtIcdLaunch L) {
-  icd_groups_body<ZL, PACK, NT, GL>(g, B, L, (int)blockIdx.x, (int)gridDim.x, (int)blockIdx.y);
-}
-
 template <int ZL, bool TAB, bool PACK, int MA = XT_MAXA, int NT = 256>
 __global__ void __launch_bounds__(NT) k_icd_lines(XtGeom g, XtIcdBuffers B, XtIcdLaunch L) {
   icd_lines_body<ZL, TAB, PACK, MA, NT>(g, B, L, (int)blockIdx.x, (int)gridDim.x,
                                         (int)blockIdx.y);
+}
+
+// ---------------------------------------------------------------------------
+// Voxel-update passes in batches of lines (the default where the A-column table
+// is kept and enough lines of a frame are in flight; the line kernel above
+// serves the rest).  One pass -- a homogeneous share or the NHICD lines, one
+// z-block parity -- runs as steps of gx lines: step t takes the lines that the
+// gx workgroups of the line kernel would each visit t-th.  All lines of a step
+// read the same error sinogram, as the line kernel's concurrent workgroups do
+// within a visit; each step sees every earlier one.
+//
+// The gx lines of a step touch every bin of a view several times (1024 lines x
+// 3.5 bins on 768 bins at 512^2), so the sinogram is streamed instead of gathered:
+// k_icd_plane holds one view's rows of e and w in LDS, applies there what the
+// previous step changed, writes e back, and sums the step's theta from LDS; e is
+// read and written once per step in whole rows, with no global atomics (the
+// line kernel's bound: one 4-byte atomic per L2 channel and clock).  The
+// generalized-Huber weight is taken once per sinogram entry instead of once per
+// (line, entry).  k_icd_step reduces the theta partials and takes the surrogate
+// step of every voxel of the step's lines, the 26 neighbours of a voxel spread
+// over its R threads.
+struct XtPass {
+  int gx;        // lines per step and frame
+  int S;         // slices of a parity (LDS slots before padding to ZC)
+  int nvc, vch;  // view chunks of a frame, views per chunk
+  int nzc;       // slot chunks of ZC
+  const int *order;    // [N_time][2][n_lines]: the iteration's line order (k_icd_order)
+  float4 *ga;          // [2][N_time][max_views][gx] column values of a step's lines, x delta_t,
+  int *gb;             // and their first bins: even and odd steps
+  float2 *part;        // [N_time][nvc][gx][S] theta1, theta2 partials
+  float *dlt;          // [N_time][gx][S] the step's changes
+  const int *cnt_col;  // [N_time][N_y*N_x] footprint entries of a line's column
+  double *st_wg;       // [workgroups of k_icd_step][4] statistics of the iteration
+  uint8_t zmap[2][64];  // slice of the k-th slot of a parity, 255 past its last
+  uint8_t zblk[2][64];  // its z-block
+  uint8_t zord[2][64];  // the slots with even slices first, each in order
+};
+
+// The homogeneous line order of an iteration, every (frame, parity) at once.
+__global__ void __launch_bounds__(256) k_icd_order(XtGeom g, XtIcdBuffers B, uint32_t seed,
+                                                   int *__restrict__ order) {
+  const int n = B.n_lines, i = blockIdx.x * 256 + threadIdx.x, f = blockIdx.y >> 1,
+            par = blockIdx.y & 1;
+  if (i >= n) return;
+  order[((size_t)f * 2 + par) * n + i] = B.lines[xt_permute(i, n, xt_order_key(seed, *B.iter, f, par))];
+}
+
+// The list a pass walks in frame f: positions lo..hi, their lines list[].  Step t's
+// j-th line is position lo + t*gx + j, or (NHICD lists, mode 1) the t-th of the j-th
+// of gx contiguous runs.
+struct XtPassList {
+  const int *list;
+  int lo, hi, steps, runs;
+};
+
+__device__ __forceinline__ XtPassList xt_pass_list(const XtGeom &g, const XtIcdBuffers &B,
+                                                   const XtIcdLaunch &L, const XtPass &P, int f,
+                                                   int par) {
+  XtPassList R;
+  if (L.mode == 1) {
+    R.list = B.nhicd_list + ((size_t)f * 2 + par) * ((size_t)g.N_y * g.N_x);
+    R.lo = 0;
+    R.hi = B.nhicd_count[f * 2 + par];
+  } else if (L.mode == 0) {
+    const int per = B.n_lines / L.K;
+    R.list = P.order + ((size_t)f * 2 + par) * B.n_lines;
+    R.lo = L.sub_iter * per;
+    R.hi = (L.sub_iter == L.K - 1) ? B.n_lines : (L.sub_iter + 1) * per;
+  } else {
+    R.list = B.lines;
+    R.lo = 0;
+    R.hi = B.n_lines;
+  }
+  R.runs = L.mode == 1;
+  R.steps = (R.hi - R.lo + P.gx - 1) / P.gx;
+  return R;
+}
+
+// the j-th line of a step, -1 if there is none
+__device__ __forceinline__ int xt_pass_line(const XtPassList &R, int gx, int step, int j) {
+  if (step < 0 || j >= gx) return -1;
+  int i = R.lo + step * gx + j, end = R.hi;
+  if (R.runs) {  // at most 2^22 lines (the plan's limit) and 1024 runs: 32-bit products
+    const uint32_t len = (uint32_t)(R.hi - R.lo);
+    i = R.lo + (int)(len * (uint32_t)j / (uint32_t)gx) + step;
+    end = R.lo + (int)(len * (uint32_t)(j + 1) / (uint32_t)gx);
+  }
+  return i < end ? R.list[i] : -1;
+}
+
+// The table columns of a step's lines, regrouped so that a view's are contiguous: a
+// line's row of the table is contiguous over the views, so k_icd_plane, which takes
+// a view at a time, would fetch a whole cache line for each 16-byte entry.  One
+// workgroup moves a tile of 16 lines x 64 views through LDS.
+__device__ __forceinline__ void xt_gather_tile(const XtGeom &g, const XtIcdBuffers &B,
+                                               const XtPass &P, const XtPassList &R, int step, int f,
+                                               int tile, char *smem) {
+  float4(*tv)[17] = (float4(*)[17])smem;
+  int(*tb)[17] = (int(*)[17])(tv + 64);
+  const int tid = threadIdx.x, nvt = (g.max_views + 63) / 64;
+  const int j0 = (tile / nvt) * 16, p0 = (tile % nvt) * 64;
+  const size_t NYX = (size_t)g.N_y * g.N_x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), p = p0 + lane;
+  float4 v4[4];
+  int b4[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int c = xt_pass_line(R, P.gx, step, j0 + wave + 4 * u);
+    v4[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    b4[u] = 0;
+    if (c >= 0 && p < g.max_views) {
+      const size_t ti = ((size_t)f * NYX + c) * g.max_views + p;
+      v4[u] = B.at_vals[ti];
+      b4[u] = B.at_first[ti];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    tv[lane][wave + 4 * u] = make_float4(v4[u].x * g.delta_t, v4[u].y * g.delta_t,
+                                         v4[u].z * g.delta_t, v4[u].w * g.delta_t);
+    tb[lane][wave + 4 * u] = b4[u];
+  }
+  __syncthreads();
+  const int jl = tid & 15, j = j0 + jl;
+  if (j >= P.gx) return;
+  const size_t row = ((size_t)(step & 1) * g.N_time + f) * g.max_views;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int pl = (tid >> 4) + 16 * u;
+    if (p0 + pl < g.max_views) {
+      P.ga[(row + p0 + pl) * P.gx + j] = tv[pl][jl];
+      P.gb[(row + p0 + pl) * P.gx + j] = tb[pl][jl];
+    }
+  }
+}
+
+// One step over the views: grid (view chunks x slot chunks, frames), threads for ZC
+// slots and LG lines at a time, I lines per thread (gx <= I * LG).
+// Applies the changes of step - 1 and sums theta for step.
+template <int ZC, int LG, int I>
+__global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers B,
+                                                                    XtIcdLaunch L, XtPass P,
+                                                                    int step) {
+  constexpr int NT = ZC * LG, NE = 12;  // NE bins of a row per thread in flight
+  constexpr int NS = (I * LG + NT - 1) / NT;  // columns a thread stages
+  const int f = blockIdx.y;
+  int tid = threadIdx.x, k = tid % ZC, lg = tid / ZC;
+  const int par = L.mode == 3 ? L.half : ((L.half ^ f) & 1);
+  const XtPassList R = xt_pass_list(g, B, L, P, f, par);
+  if (step > R.steps) return;
+  const bool prev = step > 0, cur = step < R.steps;
+  if (!prev && !cur) return;
+  // the slot chunks of a view chunk on one XCD (workgroups go to the XCDs in turn),
+  // which then share its rows and columns in L2
+  int vc, zc;
+  if (P.nvc % 8 == 0) {
+    const int lo8 = blockIdx.x & 7, hi8 = blockIdx.x >> 3;
+    zc = hi8 % P.nzc;
+    vc = (hi8 / P.nzc) * 8 + lo8;
+  } else {
+    zc = blockIdx.x % P.nzc;
+    vc = blockIdx.x / P.nzc;
+  }
+  const int nr = (g.N_r + LG - 1) / LG;  // bins of a row per thread
+  extern __shared__ float4 smem4[];
+  float4 *av = smem4;              // [I * LG] a step's column values of the view, 0 past gx
+  int *ab = (int *)(av + I * LG);  // [I * LG] its first LDS row
+  // [nr * LG + 3][ZC]: e as doubles while the changes are applied (an LDS atomic add
+  // takes 14 clocks a wave in FP64 and 194 in FP32 on gfx950), then (ws, e ws); 0 past N_r
+  float2 *pl = (float2 *)(ab + I * LG);
+  double *pd = (double *)pl;
+  const int slot = zc * ZC + k;
+  const bool on = slot < P.S && P.zmap[par][slot] != 255;
+  const int row_len = g.pm ? g.H : g.N_t;
+  const size_t plane0 = g.pm ? (size_t)par * g.N_p * g.N_r * g.H : 0;
+  const int nv = B.proj_num[f];
+  const int *vlist = B.views + (size_t)f * g.max_views;
+  const int p0 = vc * P.vch, p1 = min(nv, p0 + P.vch);
+  // this thread's lines lg, lg + LG, ...: changes to apply and sums to take
+  float dl[I], t1[I], t2[I];
+  {
+    const float *d0 = P.dlt + (size_t)f * P.gx * P.S;
+#pragma unroll
+    for (int i = 0; i < I; i++) {
+      const int j = lg + i * LG;
+      dl[i] = (prev && on && j < P.gx) ? d0[j * P.S + slot] : 0.f;
+      t1[i] = 0.f;
+      t2[i] = 0.f;
+    }
+  }
+  auto stage = [&](int st, int p) {
+    const size_t row = (((size_t)(st & 1) * g.N_time + f) * g.max_views + p) * P.gx;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const int j = tid + s * NT;
+      if (j < I * LG) {
+        av[j] = j < P.gx ? P.ga[row + j] : make_float4(0.f, 0.f, 0.f, 0.f);
+        ab[j] = j < P.gx ? P.gb[row + j] * ZC : 0;
+      }
+    }
+  };
+  // a column may reach past the last bin with zero entries: three spare rows
+  if (tid < 3 * ZC) pl[nr * LG * ZC + tid] = make_float2(0.f, 0.f);
+  const float T2 = g.T * g.T, Td = g.T * g.delta;
+  // a view's rows of e and w through buffer descriptors that end with its last bin: an
+  // offset past it, or a slot that is off, reads 0 and drops the store
+  const uint32_t row_bytes = (uint32_t)(g.N_r * row_len) * 4u;
+  uint32_t off0 =
+      on ? (uint32_t)(lg * row_len + (g.pm ? slot : P.zmap[par][slot])) * 4u : 0x80000000u;
+  const uint32_t offs = (uint32_t)(LG * row_len) * 4u;
+  for (int p = p0; p < p1; p++) {
+    // keep the compiler from hoisting every unrolled address out of this loop: they do
+    // not fit the registers and came back from scratch memory
+    asm volatile("" : "+v"(tid), "+v"(k), "+v"(lg), "+v"(off0));
+    const size_t row = plane0 + (size_t)vlist[p] * g.N_r * row_len;
+    const __amdgpu_buffer_rsrc_t rs_e =
+        __builtin_amdgcn_make_buffer_rsrc(B.e + row, 0, row_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_w =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(B.w + row), 0, row_bytes, 0x00020000);
+    auto load = [&](const __amdgpu_buffer_rsrc_t &rs, int u0, float(&v)[NE]) {
+#pragma unroll
+      for (int u = 0; u < NE; u++)
+        if (u0 + u < nr)
+          v[u] = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(rs, off0 + (uint32_t)(u0 + u) * offs, 0, 0));
+    };
+    float w8[NE];  // the first NE * LG bins' weights, loaded with their e
+    if (cur) load(rs_w, 0, w8);
+    if (prev) {
+      for (int u0 = 0; u0 < nr; u0 += NE) {
+        float e8[NE];
+        load(rs_e, u0, e8);
+#pragma unroll
+        for (int u = 0; u < NE; u++)
+          if (u0 + u < nr) pd[((u0 + u) * LG + lg) * ZC + k] = (double)e8[u];
+      }
+      stage(step - 1, p);
+      __syncthreads();
+      // e -= A * delta
+#pragma unroll
+      for (int i = 0; i < I; i++) {
+        if (dl[i] != 0.f) {
+          const float4 a = av[lg + i * LG];
+          double *q = pd + ab[lg + i * LG] + k;
+          atomicAdd(q, (double)-(a.x * dl[i]));
+          atomicAdd(q + ZC, (double)-(a.y * dl[i]));
+          atomicAdd(q + 2 * ZC, (double)-(a.z * dl[i]));
+          atomicAdd(q + 3 * ZC, (double)-(a.w * dl[i]));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // in the compiler's order the lines spill
+      }
+      __syncthreads();
+    }
+    for (int u0 = 0; u0 < nr; u0 += NE) {
+      float e8[NE];
+      if (cur && u0) load(rs_w, u0, w8);
+      if (prev) {
+#pragma unroll
+        for (int u = 0; u < NE; u++)
+          if (u0 + u < nr) {
+            e8[u] = (float)pd[((u0 + u) * LG + lg) * ZC + k];
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(e8[u]), rs_e,
+                                                  off0 + (uint32_t)(u0 + u) * offs, 0, 0);
+          }
+      } else {
+        load(rs_e, u0, e8);
+      }
+      if (cur)
+#pragma unroll
+        for (int u = 0; u < NE; u++)
+          if (u0 + u < nr) {
+            // generalized Huber weight (F/XT_ICD_update.c:577, F/XT_VoxUpdate.c:38-48,76)
+            const float wr = Td * __builtin_amdgcn_sqrtf(w8[u]) * __builtin_amdgcn_rcpf(fabsf(e8[u]));
+            const float ws = (e8[u] * e8[u] * w8[u] < T2) ? w8[u] : wr;
+            pl[((u0 + u) * LG + lg) * ZC + k] = make_float2(ws, e8[u] * ws);
+          }
+    }
+    if (cur) {
+      stage(step, p);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < I; i++) {
+        const float4 a = av[lg + i * LG];
+        const float2 *q = pl + ab[lg + i * LG] + k;
+        const float2 u0 = q[0], u1 = q[ZC], u2 = q[2 * ZC], u3 = q[3 * ZC];
+        t2[i] += a.x * (a.x * u0.x) + a.y * (a.y * u1.x) + a.z * (a.z * u2.x) + a.w * (a.w * u3.x);
+        t1[i] -= a.x * u0.y + a.y * u1.y + a.z * u2.y + a.w * u3.y;
+        if (i & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();  // the next view overwrites the plane and the columns
+  }
+  if (cur && on) {
+    int j0 = lg;
+    asm volatile("" : "+v"(j0));
+    float2 *out = P.part + ((size_t)f * P.nvc + vc) * P.gx * P.S + slot;
+#pragma unroll
+    for (int i = 0; i < I; i++)
+      if (j0 + i * LG < P.gx) out[(j0 + i * LG) * P.S] = make_float2(t1[i], t2[i]);
+  }
+}
+
+// The surrogate step (F/XT_ICD_update.c:130-179) of a step's lines: 256 threads for
+// 256 / (SP * R) lines, SP >= S slots, R threads per voxel.  Slices next to one
+// another in a z-block (blocks of several slices) are taken in red-black order.
+// x is read and written with plain accesses: what other steps wrote is visible from the
+// launch on, and lines of one step read each other's old or new x, as lines in flight
+// do.  The workgroups past the first nwg gather the next step's columns; step -1 does that
+// alone.
+template <int SP, int R>
+__global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIcdLaunch L, XtPass P,
+                                                  int step, int nwg) {
+  constexpr int PN = 256 / R, LW = PN / SP;  // (line, slot) pairs and lines of the workgroup
+  constexpr int NN = (29 + R - 1) / R;       // neighbours of a thread
+  const int f = blockIdx.y, tid = threadIdx.x;
+  const int par = L.mode == 3 ? L.half : ((L.half ^ f) & 1);
+  const XtPassList Q = xt_pass_list(g, B, L, P, f, par);
+  constexpr int kTile = 64 * 17 * (sizeof(float4) + sizeof(int));
+  constexpr int kStep = 32 + 256 * sizeof(float2) + LW * (66 + 64 + 1) * sizeof(float);
+  __shared__ __align__(16) char smem[kTile > kStep ? kTile : kStep];
+  if ((int)blockIdx.x >= nwg) {
+    if (step + 1 < Q.steps) xt_gather_tile(g, B, P, Q, step + 1, f, (int)blockIdx.x - nwg, smem);
+    return;
+  }
+  if (step >= Q.steps) return;
+  double *st = (double *)smem;              // [4]
+  float2 *red = (float2 *)(st + 4);         // [256]
+  float(*xs)[66] = (float(*)[66])(red + 256);  // [LW]
+  float(*magb)[64] = (float(*)[64])(xs + LW);  // [LW]
+  int *cl = (int *)(magb + LW);             // [LW] the workgroup's lines
+  const size_t NYX = (size_t)g.N_y * g.N_x;
+  const int iter = *B.iter, nz = g.N_z;
+  // the voxel of this thread: pair = (line l, slot kk), its share r of the neighbours;
+  // with one slice per block a parity's slices are never adjacent and one round does
+  // (with two rounds the slots of even slices come first, so that the waves of a round
+  // are full)
+  const int n_rounds = (g.pm && g.bs == 1) ? 1 : 2;
+  const int pair = tid / R, r = tid % R, l = pair / SP, ks0 = pair % SP;
+  const int kk = n_rounds == 2 && ks0 < P.S ? P.zord[par][ks0] : ks0;
+  const int j = blockIdx.x * LW + l;
+  const int c = xt_pass_line(Q, P.gx, step, j);
+  const bool vox = c >= 0 && kk < P.S && P.zmap[par][kk] != 255;
+  const int z = vox ? P.zmap[par][kk] : 0;
+  const int yy = c >= 0 ? c / g.N_x : 0, xx = c >= 0 ? c - yy * g.N_x : 0;
+  if (tid < 4) st[tid] = 0.0;
+  constexpr int TL = SP * R;  // threads of a line
+  if (tid % TL == 0) cl[l] = c;
+  for (int zz = tid % TL; zz < 64; zz += TL) {
+    xs[l][zz] = (c >= 0 && zz < nz)
+                    ? __hip_atomic_load(&B.x[((size_t)f * NYX + c) * nz + zz], __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_WAVEFRONT)
+                    : 0.f;
+    magb[l][zz] = 0.f;
+  }
+  // the thread's neighbours n = r, r + R, ...: 0..26 spatial (13 the voxel itself), 27 and
+  // 28 temporal; those in the line's own column are taken from xs when they are used
+  float nbv[NN];
+  bool nbo[NN];
+#pragma unroll
+  for (int q = 0; q < NN; q++) {
+    const int n = r + q * R;
+    const int f2 = n < 27 ? f : f + 2 * n - 55;
+    const int m = n < 27 ? n : 13;
+    const int z2 = z + m / 9 - 1, y2 = yy + (m / 3) % 3 - 1, x2 = xx + m % 3 - 1;
+    nbo[q] = vox && n < 29 && n != 13 && z2 >= 0 && z2 < nz && y2 >= 0 && y2 < g.N_y && x2 >= 0 &&
+             x2 < g.N_x && f2 >= 0 && f2 < g.N_time;
+    nbv[q] = 0.f;
+    if (nbo[q] && !(n == 4 || n == 22))
+      nbv[q] = __hip_atomic_load(&B.x[((size_t)f2 * NYX + (size_t)y2 * g.N_x + x2) * nz + z2],
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  // theta: sum of the view chunks' partials, pairs fastest (rows of gx * S float2)
+  {
+    const int pr = tid % PN, rr = tid / PN;
+    const int jj = blockIdx.x * LW + pr / SP, ks = pr % SP;
+    float2 a = make_float2(0.f, 0.f);
+    if (jj < P.gx && ks < P.S) {
+      const size_t stride = (size_t)P.gx * P.S;
+      const float2 *q = P.part + (size_t)f * P.nvc * stride + (size_t)jj * P.S + ks;
+#pragma unroll 8
+      for (int v = rr; v < P.nvc; v += R) {
+        const float2 u = q[(size_t)v * stride];
+        a.x += u.x;
+        a.y += u.y;
+      }
+    }
+    red[rr * PN + pr] = a;
+  }
+  __syncthreads();
+  float T1 = red[r * PN + l * SP + kk].x, T2 = red[r * PN + l * SP + kk].y;
+#pragma unroll
+  for (int m = 1; m < R; m <<= 1) {
+    T1 += __shfl_xor(T1, m);
+    T2 += __shfl_xor(T2, m);
+  }
+  const bool upd_ok = vox && (!B.vmask || B.vmask[((size_t)f * NYX + c) * nz + z] != 0);
+  float change = 0.f;
+  for (int round = 0; round < n_rounds; round++) {
+    const bool mine = upd_ok && (n_rounds == 1 || (z & 1) == round);
+    const float V = xs[l][z];
+    float s1 = 0.f, s2 = 0.f;
+    int pos = 0;
+    if (mine) {
+#pragma unroll
+      for (int q = 0; q < NN; q++) {
+        const int n = r + q * R;
+        if (!nbo[q]) continue;
+        const float v = n == 4 ? xs[l][z - 1] : n == 22 ? xs[l][z + 1] : nbv[q];
+        pos |= v > 0.f;
+        const bool sp = n < 27;
+        const float bq = (sp ? g.filt[n] : g.tfilt) *
+                         xt_qggmrf_ratio2(V - v, g.MRF_P, sp ? g.C_S : g.C_T,
+                                          sp ? g.Sigma_S_Q : g.Sigma_T_Q,
+                                          sp ? g.Sigma_S_Q_P : g.Sigma_T_Q_P);
+        s1 += bq * v;
+        s2 += bq;
+      }
+    }
+#pragma unroll
+    for (int m = 1; m < R; m <<= 1) {
+      s1 += __shfl_xor(s1, m);
+      s2 += __shfl_xor(s2, m);
+      pos |= __shfl_xor(pos, m);
+    }
+    // zero skipping, F/XT_VoxUpdate.c:208-232
+    if (mine && r == 0 && !(V == 0.f && iter > 1 && !pos)) {
+      const float u = (s1 + (T2 * V) - T1) / (s2 + T2);
+      float nv2 = V + g.alpha * (u - V);
+      if (g.positivity && nv2 <= 0.f) nv2 = 0.f;
+      change = nv2 - V;
+      xs[l][z] = nv2;
+      __hip_atomic_store(&B.x[((size_t)f * NYX + c) * nz + z], nv2, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_WAVEFRONT);
+      atomicAdd(&magb[l][P.zblk[par][kk]], fabsf(change));
+      if (L.count_stats) atomicAdd(&st[0], (double)fabsf(nv2));
+      atomicAdd(&st[1], 1.0);
+      atomicAdd(&st[2], (double)P.cnt_col[(size_t)f * NYX + c]);
+    }
+    __syncthreads();
+  }
+  if (r == 0 && j < P.gx && kk < P.S) P.dlt[((size_t)f * P.gx + j) * P.S + kk] = change;
+  // MagUpdateMap: the blocks of the parity (F/XT_VoxUpdate.c:128,236)
+  for (int q = tid; q < LW * g.nb; q += 256) {
+    const int ll = q / g.nb, b = q - ll * g.nb;
+    const int c2 = cl[ll];
+    if (c2 >= 0 && (b & 1) == par) B.mag_blk[((size_t)f * g.nb + b) * NYX + c2] = magb[ll][b];
+  }
+  if (tid < LW && cl[tid] >= 0) atomicAdd(&st[3], 1.0);
+  __syncthreads();
+  if (tid < 4 && st[tid] != 0.0)
+    unsafeAtomicAdd(&P.st_wg[((size_t)f * nwg + blockIdx.x) * 4 + tid], st[tid]);
+}
+
+// End of an iteration of batched passes: the workgroups' statistics into stats,
+// and each line's update magnitude over its blocks.
+__global__ void __launch_bounds__(256) k_icd_stats(const double *__restrict__ st_wg, int n,
+                                                   double *__restrict__ stats) {
+  __shared__ double s[256];
+  const int q = threadIdx.x & 3;
+  double a = 0.0;
+  for (int i = threadIdx.x >> 2; i < n; i += 64) a += st_wg[(size_t)i * 4 + q];
+  s[threadIdx.x] = a;
+  __syncthreads();
+  for (int h = 128; h >= 4; h >>= 1) {
+    if ((int)threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x < 4) stats[threadIdx.x] += s[threadIdx.x];
+}
+
+__global__ void __launch_bounds__(256) k_icd_magsum(int nb, size_t NYX, int n_time,
+                                                    const float *__restrict__ mag,
+                                                    float *__restrict__ magsum) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= NYX * n_time) return;
+  const size_t f = i / NYX, c = i % NYX;
+  float a = 0.f;
+  for (int b = 0; b < nb; b++) a += mag[(f * nb + b) * NYX + c];
+  magsum[i] = a;
+}
+
+// Footprint entries of every line's column, one wave per (frame, line).
+__global__ void __launch_bounds__(256) k_col_count(XtGeom g, const int *__restrict__ proj_num,
+                                                   const float4 *__restrict__ at_vals,
+                                                   int *__restrict__ cnt) {
+  const size_t NYX = (size_t)g.N_y * g.N_x;
+  const size_t i = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int f = blockIdx.y, lane = threadIdx.x & 63;
+  if (i >= NYX) return;
+  const float4 *row = at_vals + ((size_t)f * NYX + i) * g.max_views;
+  int n = 0;
+  for (int p = lane; p < proj_num[f]; p += 64) {
+    const float4 v = row[p];
+    n += (v.x > 0.f) + (v.y > 0.f) + (v.z > 0.f) + (v.w > 0.f);
+  }
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_down(n, o);
+  if (lane == 0) cnt[(size_t)f * NYX + i] = n;
 }
 
 // One slab of a batch launch: its state, its launch parameters, its workgroups

@@ -68,7 +68,7 @@ int xt_report_error(int code, const char *fmt, ...) {
     if (_rc != XT_OK) return _rc; \
   } while (0)
 
-static double g_opt[20] = {0, 0, 0, 0, 761521, 0, 0, 1, 0, 1, 1, 1, 1, 0, 1, 0, 0, 0, 0, 1};  // XT_OPT_*
+static double g_opt[21] = {0, 0, 0, 0, 761521, 0, 0, 1, 0, 1, 1, 1, 1, 0, 1, 0, 0, 0, 0, 1, 0};  // XT_OPT_*
 // bumped whenever an option changes value: a captured iteration graph (which
 // froze the options it was recorded under) is recaptured when it differs
 static uint64_t g_opt_gen = 1;
@@ -78,20 +78,21 @@ extern "C" const char *xt_last_error(void) { return g_err; }
 extern "C" const char *xt_version(void) { return "libxt_hip gfx950 Real_t=" XT_REAL_NAME; }
 
 extern "C" int xt_set_option(int option, double value) {
-  if (option < 1 || option > 19) return set_err(XT_E_ARG, "unknown option %d", option);
+  if (option < 1 || option > 20) return set_err(XT_E_ARG, "unknown option %d", option);
   if (option == XT_OPT_LINE_THREADS && value != 0 && value != 64 && value != 256)
     return set_err(XT_E_ARG, "XT_OPT_LINE_THREADS must be 0, 64 or 256");
-  // groups of 2 or 4 lines (k_icd_groups) are switched off: their first run on the
-  // GPU took a memory fault whose cause is not found (the kernel is memory-safe by
-  // construction and passes the per-voxel checks in a CPU build of this file)
+  // updates in groups of 2 or 4 lines are not in this build: their first run on the GPU
+  // took a memory fault whose cause is not found
   if (option == XT_OPT_LINE_GROUP && value != 1)
     return set_err(XT_E_ARG, "XT_OPT_LINE_GROUP: only 1 (single lines) is enabled in this build");
+  if (option == XT_OPT_PASS && value != 0 && value != 1 && value != 2)
+    return set_err(XT_E_ARG, "XT_OPT_PASS must be 0, 1 or 2");
   if (g_opt[option] != value) g_opt_gen++;
   g_opt[option] = value;
   return XT_OK;
 }
 extern "C" double xt_get_option(int option) {
-  return (option >= 1 && option <= 19) ? g_opt[option] : NAN;
+  return (option >= 1 && option <= 20) ? g_opt[option] : NAN;
 }
 
 static std::string run_path(const char *name) {
@@ -303,10 +304,6 @@ struct xt_icd_state {
   int *views = nullptr, *proj_num = nullptr, *view_frame = nullptr;
   int *vpos = nullptr;  // each view's position in its frame's list
   int *lines = nullptr, *nhicd_list = nullptr, *nhicd_count = nullptr;
-  // the homogeneous passes' line groups: 1 x 2 tiles (groups2) and 2 x 2 tiles
-  // (groups4) of the line list, members first and -1 after them
-  int *groups2 = nullptr, *groups4 = nullptr;
-  int n_groups2 = 0, n_groups4 = 0;
   int *nhicd_chunk = nullptr;  // NHICD list compaction: lines per chunk of each map
   uint8_t *line_mask = nullptr;
   uint8_t *nhicd_flag = nullptr, *nhicd_blk = nullptr;
@@ -329,6 +326,20 @@ struct xt_icd_state {
   uint64_t lines_gen = 1;       // bumped when the line list or its NHICD shares change
   int64_t graph_launches = 0;   // voxel-update launches in the captured iteration
   int off_nch = 1, off_chunk = 1, off_nblk = 1;
+  // batched passes (k_icd_plane, k_icd_step): what they are launched with, for up
+  // to pass_gx lines per step; the buffers are the state's, so every stream and
+  // batch branch has its own
+  bool pass_ok = false;
+  XtPass pass{};
+  int pass_gx = 0, pass_zc = 0;
+  int nsel_max = 0;  // most lines an NHICD list of the per-parity rule can hold
+  int *order = nullptr, *cnt_col = nullptr;
+  float2 *pass_part = nullptr;
+  float4 *pass_ga = nullptr;
+  int *pass_gb = nullptr;
+  float *pass_dlt = nullptr;
+  double *st_wg = nullptr;
+  int st_n = 0;
   // statistics
   double total_updates = 0, total_foot = 0, total_visits = 0, icd_ms = 0, last_cost = NAN,
          stop_pct = NAN;
@@ -351,7 +362,8 @@ static void free_state(xt_icd_state *s) {
                   s->magpar,
                   s->red_wg,   s->scal,       s->off_part, s->off_numden, s->off_wg,
                   s->at_vals,  s->at_first,   s->iter_dev, s->pc_tmp, s->vmask, s->vsc_st,
-                  s->vsc_hist, s->groups2, s->groups4};
+                  s->vsc_hist, s->order, s->cnt_col,
+                  s->pass_part, s->pass_dlt, s->st_wg, s->pass_ga, s->pass_gb};
   if (s->graph_exec) (void)hipGraphExecDestroy(s->graph_exec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   for (void *b : bufs)
@@ -425,23 +437,7 @@ static void icd_launch_nt(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B
                           const XtIcdLaunch &L, int gx, size_t lds) {
   const dim3 grid(gx, g.N_time), block(NT);
   const bool pack = icd_packable(g, ZL, L);
-  if (B.gl == 2 || B.gl == 4) {  // groups of lines, from the table
-    if (B.gl == 2) {
-      if (pack)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_groups<ZL, true, NT, 2>), grid, block, lds, st, g,
-                           B, L);
-      else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_groups<ZL, false, NT, 2>), grid, block, lds, st, g,
-                           B, L);
-    } else {
-      if (pack)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_groups<ZL, true, NT, 4>), grid, block, lds, st, g,
-                           B, L);
-      else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_groups<ZL, false, NT, 4>), grid, block, lds, st, g,
-                           B, L);
-    }
-  } else if (g.wide) {  // never with the table (it holds four bins per column)
+  if (g.wide) {  // never with the table (it holds four bins per column)
     if (pack)
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_lines<ZL, false, true, XT_MAXA_WIDE, NT>), grid,
                          block, lds, st, g, B, L);
@@ -497,41 +493,222 @@ static XtIcdBuffers buffers_of(xt_icd_state *s) {
   B.at_first = s->at_first;
   B.iter = s->iter_dev;
   B.vmask = s->vmask;
-  B.groups = nullptr;
-  B.n_groups = 0;
-  B.gl = 1;
   return B;
 }
 
 // One voxel-update launch over a range of lines; gx workgroups per frame.
-// Lines per workgroup item of the voxel-update launches (XT_OPT_LINE_GROUP): 2
-// or 4 with the A-column table and slices of one detector row, else 1.
-static int line_group(const xt_icd_state *s) {
-  const int gl = (int)g_opt[XT_OPT_LINE_GROUP];
-  if ((gl != 2 && gl != 4) || !s->at_vals || s->g.wide || s->g.pc || s->g.zo != 1) return 1;
-  return gl;
+// ---- batched passes
+constexpr int kPassRow = 64;  // lines of a k_icd_plane workgroup at a time
+
+static int pass_rows(int gx) {  // lines per thread, the variant's
+  const int I = (gx + kPassRow - 1) / kPassRow;
+  return I <= 1 ? 1 : I <= 2 ? 2 : I <= 4 ? 4 : I <= 8 ? 8 : 16;
 }
 
-static size_t group_lds_bytes(const XtGeom &g, int ZL, int gl, int nt) {
-  return (size_t)g.max_views * sizeof(int) + 2 * (size_t)nt * sizeof(float) +
-         (size_t)(13 + gl) * ZL * sizeof(float) + 64 * sizeof(float);
+static size_t pass_lds(const XtGeom &g, int zc, int gx) {
+  return (size_t)pass_rows(gx) * kPassRow * (sizeof(float4) + sizeof(int)) +
+         (size_t)((g.N_r + kPassRow - 1) / kPassRow * kPassRow + 3) * zc * sizeof(float2);
+}
+
+// f(kernel, threads) on the k_icd_plane instantiation for zc slots and gx lines
+template <int ZC, typename F>
+static void plane_pick(int gx, F f) {
+  constexpr int LG = kPassRow;
+  const int I = pass_rows(gx);
+  if (I <= 1) f(k_icd_plane<ZC, LG, 1>, ZC * LG);
+  else if (I <= 2) f(k_icd_plane<ZC, LG, 2>, ZC * LG);
+  else if (I <= 4) f(k_icd_plane<ZC, LG, 4>, ZC * LG);
+  else if (I <= 8) f(k_icd_plane<ZC, LG, 8>, ZC * LG);
+  else f(k_icd_plane<ZC, LG, 16>, ZC * LG);
+}
+
+template <typename F>
+static void plane_pick(int zc, int gx, F f) {
+  if (zc == 4) plane_pick<4>(gx, f);
+  else if (zc == 8) plane_pick<8>(gx, f);
+  else plane_pick<16>(gx, f);
+}
+
+// slots of a line and threads per voxel of k_icd_step: 16 threads share a voxel's
+// neighbours while the workgroups of a step all fit the chip at once (512^2 x 32: 246 ms
+// for two iterations against 249 with 8), fewer beyond that (16 frames of 512 lines x 8
+// slots: 230 ms against 237 for four iterations)
+static int step_slots(int S) { return S <= 4 ? 4 : S <= 8 ? 8 : S <= 16 ? 16 : S <= 32 ? 32 : 64; }
+
+static int step_threads(int S, int lines) {
+  const int sp = step_slots(S);
+  return sp <= 16 && (size_t)lines * sp * 16 <= 256 * 1024 ? 16 : sp <= 16 ? 8 : 4;
+}
+
+static int step_lines(int S, int lines) { return 256 / (step_slots(S) * step_threads(S, lines)); }
+
+// step -1 only gathers the columns of step 0; the last step gathers none
+template <int SP, int R>
+static void step_go(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B, const XtIcdLaunch &L,
+                    const XtPass &P, int step, bool gather) {
+  constexpr int lw = 256 / (SP * R);
+  const int nwg = step < 0 ? 0 : (P.gx + lw - 1) / lw;
+  const int ng = gather ? ((P.gx + 15) / 16) * ((g.max_views + 63) / 64) : 0;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R>), dim3(nwg + ng, g.N_time), dim3(256), 0, st, g,
+                     B, L, P, step, nwg);
+}
+
+static void step_launch(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B, const XtIcdLaunch &L,
+                        const XtPass &P, int step, bool gather) {
+  const int sp = step_slots(P.S), r = step_threads(P.S, P.gx * g.N_time);
+  if (sp == 4 && r == 16) step_go<4, 16>(st, g, B, L, P, step, gather);
+  else if (sp == 4) step_go<4, 8>(st, g, B, L, P, step, gather);
+  else if (sp == 8 && r == 16) step_go<8, 16>(st, g, B, L, P, step, gather);
+  else if (sp == 8) step_go<8, 8>(st, g, B, L, P, step, gather);
+  else if (sp == 16 && r == 16) step_go<16, 16>(st, g, B, L, P, step, gather);
+  else if (sp == 16) step_go<16, 8>(st, g, B, L, P, step, gather);
+  else if (sp == 32) step_go<32, 4>(st, g, B, L, P, step, gather);
+  else step_go<64, 4>(st, g, B, L, P, step, gather);
+}
+
+// (re)allocates a buffer of the batched passes; non-zero when the memory is not there
+template <typename T>
+static int pass_alloc(T **p, size_t n) {
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  const hipError_t e = hipMalloc((void **)p, (n ? n : 1) * sizeof(T));
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+  }
+  return e != hipSuccess;
+}
+
+// Plans the batched passes for up to gx lines per step and allocates their buffers;
+// pass_ok stays false where they do not apply (the line kernel then runs).
+static int plan_pass(xt_icd_state *s, int gx) {
+  const XtGeom &g = s->g;
+  s->pass_ok = false;
+  if (!s->at_vals || g.wide || g.pc || g.zo != 1 || gx < 1 || gx > 1024 ||
+      s->NYX > ((size_t)1 << 22))
+    return XT_OK;
+  XtPass &P = s->pass;
+  memset(&P, 0, sizeof P);
+  const int bs = g.N_z / g.nb;
+  int n[2] = {0, 0};
+  for (int z = 0; z < g.N_z; z++) {
+    int b = bs > 0 ? z / bs : g.nb - 1;
+    if (b >= g.nb) b = g.nb - 1;
+    P.zblk[b & 1][n[b & 1]] = (uint8_t)b;
+    P.zmap[b & 1][n[b & 1]++] = (uint8_t)z;
+  }
+  P.S = std::max(n[0], n[1]);
+  for (int q = 0; q < 2; q++) {
+    for (int k = n[q]; k < 64; k++) P.zmap[q][k] = 255;
+    int m = 0;
+    for (int odd = 0; odd < 2; odd++)
+      for (int k = 0; k < P.S; k++)
+        if ((P.zmap[q][k] & 1) == odd) P.zord[q][m++] = (uint8_t)k;
+  }
+  // as many slots of a bin together as there are (up to 16: a wave's LDS accesses then
+  // fall into 4 runs of 128 bytes instead of 16 of 32; 512^2 x 32, two iterations: 247 ms
+  // with 16 slots, 261 with 8, 345 with 4), while the rows fit the LDS
+  int zc = P.S <= 4 ? 4 : P.S <= 8 ? 8 : 16;
+  int lds_max = 0;
+  (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->dev);
+  while (zc > 4 && pass_lds(g, zc, gx) > (size_t)lds_max) zc /= 2;
+  const size_t lds = pass_lds(g, zc, gx);
+  if (lds > (size_t)lds_max) return XT_OK;
+  s->pass_zc = zc;
+  P.nzc = (P.S + zc - 1) / zc;
+  // one or two workgroups per CU, by LDS: with half of them the same slab takes 321 ms
+  const int occ = std::max(1, std::min({(int)(160 * 1024 / lds), 2048 / (zc * kPassRow), 2}));
+  const int target = 256 * occ;
+  P.vch = std::max(1, (g.N_time * g.max_views * P.nzc + target - 1) / target);
+  P.nvc = (g.max_views + P.vch - 1) / P.vch;
+  s->pass_gx = gx;
+  const int lw = step_lines(P.S, gx * g.N_time);
+  s->st_n = ((gx + lw - 1) / lw) * g.N_time;
+  if (lds > 64 * 1024) {
+    hipError_t e = hipSuccess;
+    for (int n = kPassRow; n <= 1024; n *= 2)  // every lines-per-thread variant
+      plane_pick(zc, n, [&](auto k, int) {
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      });
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return XT_OK;
+    }
+  }
+  const size_t fg = (size_t)g.N_time * gx, fv = (size_t)2 * fg * g.max_views;
+  // without the memory for them the line kernel serves
+  if (pass_alloc(&s->pass_part, fg * P.nvc * P.S) || pass_alloc(&s->pass_dlt, fg * P.S) ||
+      pass_alloc(&s->pass_ga, fv) || pass_alloc(&s->pass_gb, fv) ||
+      pass_alloc(&s->st_wg, (size_t)s->st_n * 4) ||
+      (!s->order && pass_alloc(&s->order, (size_t)g.N_time * 2 * s->NYX)))
+    return XT_OK;
+  if (!s->cnt_col) {
+    if (pass_alloc(&s->cnt_col, (size_t)g.N_time * s->NYX)) return XT_OK;
+    hipLaunchKernelGGL(k_col_count, dim3((unsigned)((s->NYX + 3) / 4), g.N_time), dim3(256), 0, s->st,
+                       g, s->proj_num, s->at_vals, s->cnt_col);
+    XT_HIP(hipGetLastError());
+  }
+  P.order = s->order;
+  P.part = s->pass_part;
+  P.dlt = s->pass_dlt;
+  P.ga = s->pass_ga;
+  P.gb = s->pass_gb;
+  P.cnt_col = s->cnt_col;
+  P.st_wg = s->st_wg;
+  s->pass_ok = true;
+  return XT_OK;
+}
+
+// steps of a pass at gx lines per step (the host's bound: an NHICD list may be shorter)
+static int pass_steps(const xt_icd_state *s, int mode, int sub_iter, int K, int gx) {
+  int n = s->n_masked;
+  if (mode == 0) n = sub_iter == K - 1 ? n - (n / K) * sub_iter : n / K;
+  if (mode == 1) n = s->nsel_max;
+  return (n + gx - 1) / gx;
+}
+
+// Whether a pass of this mode runs in batches.  NHICD lists of the per-block rule have
+// no useful bound on their length.  From 16 lines in flight on, batches are the
+// faster from 32^2 x 4 (10.4 ms for two iterations against 12.7) to 512^2 x 32 (246
+// against 382); a pass of more than 128 steps (lines in flight set far below the
+// default) would be thousands of small launches.
+static bool pass_batched(const xt_icd_state *s, int mode, int gx) {
+  if (!s->pass_ok || g_opt[XT_OPT_PASS] == 1 || gx < 1 || gx > s->pass_gx) return false;
+  if (mode == 1 && g_opt[XT_OPT_NHICD_LINES] == 0) return false;
+  if (mode == 2) return false;
+  if (mode == 3) return g_opt[XT_OPT_PASS] == 2;
+  const int steps = pass_steps(s, mode, s->K - 1, s->K, gx);
+  return (g_opt[XT_OPT_PASS] == 2 || (gx >= 16 && (steps <= 64 || gx >= 1024))) && steps <= 128;
+}
+
+// Launches of an iteration's voxel updates: a captured graph is kept to a few thousand
+// nodes (512^2 lines: 2160), longer iterations are enqueued.
+static bool graph_fits(const xt_icd_state *s) {
+  if (!pass_batched(s, 0, s->conc)) return true;
+  return 4 * s->K * (2 * pass_steps(s, 0, s->K - 1, s->K, s->conc) + 2) <= 4096;
+}
+
+static int launch_pass(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
+  const XtIcdBuffers B = buffers_of(s);
+  XtPass P = s->pass;
+  P.gx = gx;
+  const int steps = pass_steps(s, L.mode, L.sub_iter, L.K, gx);
+  if (steps > 0) step_launch(s->st, s->g, B, L, P, -1, true);
+  for (int t = 0; t <= steps && steps > 0; t++) {
+    plane_pick(s->pass_zc, gx, [&](auto k, int nt) {
+      hipLaunchKernelGGL(k, dim3(P.nvc * P.nzc, s->g.N_time), dim3(nt),
+                         pass_lds(s->g, s->pass_zc, gx), s->st, s->g, B, L, P, t);
+    });
+    if (t < steps) step_launch(s->st, s->g, B, L, P, t, t + 1 < steps);
+  }
+  XT_HIP(hipGetLastError());
+  return XT_OK;
 }
 
 static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
   XtIcdBuffers B = buffers_of(s);
   size_t lds = icd_lds_bytes(s->g, s->ZL, B.at_vals != nullptr, s->nt);
-  const int gl = line_group(s);
-  if (gl > 1) {
-    B.gl = gl;
-    B.groups = gl == 2 ? s->groups2 : s->groups4;
-    B.n_groups = gl == 2 ? s->n_groups2 : s->n_groups4;
-    lds = group_lds_bytes(s->g, s->ZL, gl, s->nt);
-    if (L.mode == 0) {  // no more workgroups than the sub-iteration has groups
-      const int per = B.n_groups / L.K;
-      const int share = (L.sub_iter == L.K - 1) ? B.n_groups - L.sub_iter * per : per;
-      if (gx > share) gx = share;
-    }
-  }
   if (gx < 1) gx = 1;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (s->timing) {
@@ -546,6 +723,12 @@ static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
     e1 = s->ev[s->ev_used + 1];
     s->ev_used += 2;
     XT_HIP(hipEventRecord(e0, s->st));
+  }
+  if (pass_batched(s, L.mode, gx)) {
+    XT_TRY(launch_pass(s, L, gx));
+    if (s->timing) XT_HIP(hipEventRecord(e1, s->st));
+    s->launches++;
+    return XT_OK;
   }
   if (s->g.pc) {
     const dim3 grid(gx, s->g.N_time), block(256);
@@ -569,6 +752,15 @@ static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
   XT_HIP(hipGetLastError());
   if (s->timing) XT_HIP(hipEventRecord(e1, s->st));
   s->launches++;
+  return XT_OK;
+}
+
+static int launch_order(xt_icd_state *s) {
+  const XtIcdBuffers B = buffers_of(s);
+  if (B.n_lines > 0)
+    hipLaunchKernelGGL(k_icd_order, dim3((B.n_lines + 255) / 256, s->g.N_time * 2), dim3(256), 0, s->st,
+                       s->g, B, (uint32_t)(int64_t)g_opt[XT_OPT_SEED], s->order);
+  XT_HIP(hipGetLastError());
   return XT_OK;
 }
 
@@ -660,37 +852,6 @@ static int vsc_select(xt_icd_state *s) {
 // lines read each other's stale error sinogram; a CPU simulation of that
 // coupling kept the reference's trajectory up to ~6% of the lines at once
 // and diverged at 25%), or XT_OPT_LINES when set.
-// The groups of the homogeneous passes (XT_OPT_LINE_GROUP 2 and 4): the listed
-// lines of each 1 x 2 and of each 2 x 2 tile of the image, tiles in raster order.
-static int build_groups(xt_icd_state *s, const std::vector<int> &lines) {
-  const int NX = s->g.N_x, NY = s->g.N_y;
-  std::vector<uint8_t> in(s->NYX, 0);
-  for (int c : lines) in[c] = 1;
-  for (int gl : {2, 4}) {
-    const int th = gl == 4 ? 2 : 1;  // tile rows
-    std::vector<int> grp;
-    for (int ty = 0; ty < NY; ty += th)
-      for (int tx = 0; tx < NX; tx += 2) {
-        int mem[4], n = 0;
-        for (int dy = 0; dy < th; dy++)
-          for (int dx = 0; dx < 2; dx++) {
-            const int y = ty + dy, x = tx + dx;
-            if (y < NY && x < NX && in[(size_t)y * NX + x]) mem[n++] = y * NX + x;
-          }
-        if (n == 0) continue;
-        for (int m = 0; m < gl; m++) grp.push_back(m < n ? mem[m] : -1);
-      }
-    int *&dst = gl == 2 ? s->groups2 : s->groups4;
-    if (dst) (void)hipFree(dst);
-    dst = nullptr;
-    XT_TRY(dev_alloc(&dst, grp.empty() ? 1 : grp.size()));
-    if (!grp.empty())
-      XT_HIP(hipMemcpy(dst, grp.data(), grp.size() * sizeof(int), hipMemcpyHostToDevice));
-    (gl == 2 ? s->n_groups2 : s->n_groups4) = (int)(grp.size() / gl);
-  }
-  return XT_OK;
-}
-
 static int setup_lines(xt_icd_state *s, const std::vector<int> &masked) {
   int conc = (int)g_opt[XT_OPT_LINES];
   if (conc <= 0) {
@@ -712,7 +873,7 @@ static int setup_lines(xt_icd_state *s, const std::vector<int> &masked) {
     XT_HIP(hipMemcpy(s->lines, masked.data(), masked.size() * sizeof(int), hipMemcpyHostToDevice));
   XT_HIP(hipMemcpy(s->line_mask, in.data(), s->NYX, hipMemcpyHostToDevice));
   XT_HIP(hipMemset(s->nhicd_count, 0, s->g.N_time * 2 * sizeof(int)));
-  return build_groups(s, masked);
+  return XT_OK;
 }
 
 // the detector-table kernel reduces angles by repeated subtraction of pi/2
@@ -1093,10 +1254,10 @@ static int select_edges(xt_icd_state *s) {
   }
   for (int &n : ns) n /= s->K;
   for (int &n : np) n /= s->K;
+  s->nsel_max = *std::max_element(np.begin(), np.end());
   s->n_masked = (int)lines.size();
   if (!lines.empty())
     XT_HIP(hipMemcpy(s->lines, lines.data(), lines.size() * sizeof(int), hipMemcpyHostToDevice));
-  XT_TRY(build_groups(s, lines));
   XT_HIP(hipMemcpy(s->nsel, ns.data(), ns.size() * sizeof(int), hipMemcpyHostToDevice));
   XT_HIP(hipMemcpy(s->nsel_par, np.data(), np.size() * sizeof(int), hipMemcpyHostToDevice));
   drop_graph(s);
@@ -1147,6 +1308,7 @@ static int create_impl(Sinogram *S, ScannedObject *O, TomoInputs *T, xt_icd_stat
       if (xc * xc + yc * yc < T->radius_obj * T->radius_obj) masked.push_back(j * g.N_x + k);
     }
   s->n_masked = (int)masked.size();
+  s->nsel_max = s->n_masked / s->K;
   // split the sinogram by z-block parity when the passes can pack their lanes
   if (g_opt[XT_OPT_PACK] != 0 && !g.pc && g.zo == 1 && g.nb % 2 == 0 && g.N_z % g.nb == 0 &&
       g.N_t % 2 == 0) {
@@ -1243,8 +1405,17 @@ static int create_impl(Sinogram *S, ScannedObject *O, TomoInputs *T, xt_icd_stat
   if (hipStreamSynchronize(s->st) != hipSuccess)
     return fail(set_err(XT_E_HIP, "initialisation kernels failed"));
   s->nt = ((int)g_opt[XT_OPT_LINE_THREADS] == 64 && !g.pc) ? 64 : 256;
-  if (g_opt[XT_OPT_AUTOTUNE] != 0 && g_opt[XT_OPT_LINES] == 0 && (rc = icd_autotune(s)))
-    return fail(rc);
+  if (g_opt[XT_OPT_PASS] != 1 && (rc = plan_pass(s, s->conc))) return fail(rc);
+  // the line kernel's launch shape; batched passes take every line in flight (fewer only
+  // make more steps), but the per-block rule's NHICD passes still run on it
+  if ((!pass_batched(s, 0, s->conc) || g_opt[XT_OPT_NHICD_LINES] == 0) &&
+      g_opt[XT_OPT_AUTOTUNE] != 0 && g_opt[XT_OPT_LINES] == 0) {
+    const bool ok = s->pass_ok;
+    s->pass_ok = false;
+    rc = icd_autotune(s);
+    s->pass_ok = ok;
+    if (rc) return fail(rc);
+  }
   *out = s;
   return XT_OK;
 }
@@ -1299,6 +1470,12 @@ extern "C" int xt_icd_cost(xt_icd_state *s, double *cost) {
 // under capture): the schedule of F/XT_ICD_update.c:794-882.
 static int enqueue_iteration(xt_icd_state *s, bool nhicd) {
   hipLaunchKernelGGL(k_begin_iteration, dim3(1), dim3(64), 0, s->st, s->iter_dev, s->stats, 8);
+  const bool batched = pass_batched(s, 0, s->conc);
+  if (batched) {
+    hipLaunchKernelGGL(k_zero_f64, dim3((s->st_n * 4 + 255) / 256), dim3(256), 0, s->st, s->st_wg,
+                       s->st_n * 4);
+    XT_TRY(launch_order(s));
+  }
   XtIcdLaunch L;
   L.zorder = 0;
   L.K = s->K;
@@ -1327,6 +1504,12 @@ static int enqueue_iteration(xt_icd_state *s, bool nhicd) {
         if (s->update_offset > 1) XT_TRY(offset_update(s));
       }
     }
+  }
+  if (batched) {
+    hipLaunchKernelGGL(k_icd_stats, dim3(1), dim3(256), 0, s->st, s->st_wg, s->st_n, s->stats);
+    hipLaunchKernelGGL(k_icd_magsum, dim3((unsigned)((s->NYX * s->g.N_time + 255) / 256)), dim3(256), 0,
+                       s->st, s->g.nb, s->NYX, s->g.N_time, s->mag_blk, s->magsum);
+    XT_HIP(hipGetLastError());
   }
   return XT_OK;
 }
@@ -1374,7 +1557,7 @@ static int iterate_one(xt_icd_state *s) {
   // once and replay it (no memset nodes; the iteration number lives on the device)
   // (per-launch timing needs eager launches: HIP does not report elapsed times
   // of events recorded inside a graph replay)
-  const bool use_graph = g_opt[XT_OPT_GRAPH] != 0 && Iter > 1 && !s->timing;
+  const bool use_graph = g_opt[XT_OPT_GRAPH] != 0 && Iter > 1 && !s->timing && graph_fits(s);
   if (use_graph) {
     if (s->graph_exec && s->graph_opt_gen != g_opt_gen) drop_graph(s);
     if (!s->graph_exec) {
@@ -1824,7 +2007,8 @@ extern "C" int xt_icd_batch_iterate(xt_icd_batch *b, int32_t n_iter) {
     bool graphable = g_opt[XT_OPT_GRAPH] != 0;
     for (size_t i = 0; i < b->s.size(); i++) {
       iters[i] = ++b->s[i]->iter;
-      graphable = graphable && iters[i] > 1 && !b->s[i]->timing && b->s[i]->update_var != 1;
+      graphable = graphable && iters[i] > 1 && !b->s[i]->timing && b->s[i]->update_var != 1 &&
+                  graph_fits(b->s[i]);
     }
     // the batch stream starts after whatever the slabs' own streams hold
     for (size_t i = 0; i < b->s.size(); i++) {
@@ -2578,7 +2762,18 @@ static int update_lines_impl(Sinogram *S, ScannedObject *O, TomoInputs *T, Real_
   L.seed = 0;
   L.count_stats = 1;
   L.zorder = parity < 0 ? 1 : 0;
-  XT_TRY(launch_icd(s, L, 1));
+  int gx = 1;
+  if (parity >= 0 && g_opt[XT_OPT_PASS] == 2) {  // batches of XT_OPT_LINES listed lines
+    gx = std::max(1, (int)g_opt[XT_OPT_LINES]);
+    XT_TRY(plan_pass(s, gx));
+    if (s->st_wg) XT_HIP(hipMemset(s->st_wg, 0, (size_t)s->st_n * 4 * sizeof(double)));
+  }
+  XT_TRY(launch_icd(s, L, gx));
+  if (pass_batched(s, L.mode, gx)) {
+    hipLaunchKernelGGL(k_icd_stats, dim3(1), dim3(256), 0, s->st, s->st_wg, s->st_n, s->stats);
+    hipLaunchKernelGGL(k_icd_magsum, dim3((unsigned)((s->NYX + 255) / 256)), dim3(256), 0, s->st, g.nb,
+                       s->NYX, g.N_time, s->mag_blk, s->magsum);
+  }
   XT_HIP(hipStreamSynchronize(s->st));
   if (g.pm) {
     float *tmp = nullptr;
