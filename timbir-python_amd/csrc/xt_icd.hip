@@ -668,6 +668,17 @@ static int pass_steps(const xt_icd_state *s, int mode, int sub_iter, int K, int 
   return (n + gx - 1) / gx;
 }
 
+// Lines of a step for gx lines in flight.  A line of a step misses the changes of the
+// step's earlier lines, half of them on average, one of the line kernel's nearly all that
+// are in flight; over several frames 3/2 times the lines per step follow the line
+// kernel's iterates most closely (16 frames of 256^2 x 16 with 512 lines in flight, four
+// iterations: MAP cost 7.577e8 and ring offsets 2.2e-3 apart with 768 per step, 7.568e8
+// and 3.7e-3 with 512; two runs of the line kernel 7.576e8 and 2.1e-3), on single frames
+// the same number does.
+static int pass_lines(const xt_icd_state *s, int gx) {
+  return s->g.N_time > 1 ? std::min(1024, gx + gx / 2) : gx;
+}
+
 // Whether a pass of this mode runs in batches.  NHICD lists of the per-block rule have
 // no useful bound on their length.  From 16 lines in flight on, batches are the
 // faster from 32^2 x 4 (10.4 ms for two iterations against 12.7) to 512^2 x 32 (246
@@ -685,8 +696,8 @@ static bool pass_batched(const xt_icd_state *s, int mode, int gx) {
 // Launches of an iteration's voxel updates: a captured graph is kept to a few thousand
 // nodes (512^2 lines: 2160), longer iterations are enqueued.
 static bool graph_fits(const xt_icd_state *s) {
-  if (!pass_batched(s, 0, s->conc)) return true;
-  return 4 * s->K * (2 * pass_steps(s, 0, s->K - 1, s->K, s->conc) + 2) <= 4096;
+  if (!pass_batched(s, 0, pass_lines(s, s->conc))) return true;
+  return 4 * s->K * (2 * pass_steps(s, 0, s->K - 1, s->K, pass_lines(s, s->conc)) + 2) <= 4096;
 }
 
 static int launch_pass(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
@@ -724,8 +735,8 @@ static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
     s->ev_used += 2;
     XT_HIP(hipEventRecord(e0, s->st));
   }
-  if (pass_batched(s, L.mode, gx)) {
-    XT_TRY(launch_pass(s, L, gx));
+  if (pass_batched(s, L.mode, pass_lines(s, gx))) {
+    XT_TRY(launch_pass(s, L, pass_lines(s, gx)));
     if (s->timing) XT_HIP(hipEventRecord(e1, s->st));
     s->launches++;
     return XT_OK;
@@ -1405,10 +1416,10 @@ static int create_impl(Sinogram *S, ScannedObject *O, TomoInputs *T, xt_icd_stat
   if (hipStreamSynchronize(s->st) != hipSuccess)
     return fail(set_err(XT_E_HIP, "initialisation kernels failed"));
   s->nt = ((int)g_opt[XT_OPT_LINE_THREADS] == 64 && !g.pc) ? 64 : 256;
-  if (g_opt[XT_OPT_PASS] != 1 && (rc = plan_pass(s, s->conc))) return fail(rc);
+  if (g_opt[XT_OPT_PASS] != 1 && (rc = plan_pass(s, pass_lines(s, s->conc)))) return fail(rc);
   // the line kernel's launch shape; batched passes take every line in flight (fewer only
   // make more steps), but the per-block rule's NHICD passes still run on it
-  if ((!pass_batched(s, 0, s->conc) || g_opt[XT_OPT_NHICD_LINES] == 0) &&
+  if ((!pass_batched(s, 0, pass_lines(s, s->conc)) || g_opt[XT_OPT_NHICD_LINES] == 0) &&
       g_opt[XT_OPT_AUTOTUNE] != 0 && g_opt[XT_OPT_LINES] == 0) {
     const bool ok = s->pass_ok;
     s->pass_ok = false;
@@ -1470,7 +1481,7 @@ extern "C" int xt_icd_cost(xt_icd_state *s, double *cost) {
 // under capture): the schedule of F/XT_ICD_update.c:794-882.
 static int enqueue_iteration(xt_icd_state *s, bool nhicd) {
   hipLaunchKernelGGL(k_begin_iteration, dim3(1), dim3(64), 0, s->st, s->iter_dev, s->stats, 8);
-  const bool batched = pass_batched(s, 0, s->conc);
+  const bool batched = pass_batched(s, 0, pass_lines(s, s->conc));
   if (batched) {
     hipLaunchKernelGGL(k_zero_f64, dim3((s->st_n * 4 + 255) / 256), dim3(256), 0, s->st, s->st_wg,
                        s->st_n * 4);
