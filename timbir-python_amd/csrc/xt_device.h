@@ -1772,69 +1772,91 @@ __global__ void k_offset_partial(XtGeom g, const float *__restrict__ e, const fl
   part[((size_t)ch * 2 + 1) * NRT + rt] = den;
 }
 
-__global__ void k_offset_combine(XtGeom g, int nch, const double *__restrict__ part,
-                                 const float *__restrict__ d, double *__restrict__ numden /*[2][NRT]*/,
-                                 double *__restrict__ wg_sums /*[nblk][2]*/) {
+// Sums of a pixel's view chunks, and per workgroup the two sums that gamma is made of.
+// PX pixels and 256 / PX chunk groups a workgroup: 32 pixels where there are 8 chunks or
+// more (small detectors; with one thread walking all chunks of a pixel the kernel took
+// 37 us on 192 x 8 pixels in 171 chunks, 5 us with 8 groups and chunks of 8 views or more).
+template <int PX>
+__global__ void __launch_bounds__(256) k_offset_combine(XtGeom g, int nch,
+                                                        const double *__restrict__ part,
+                                                        const float *__restrict__ d,
+                                                        double *__restrict__ numden /*[2][NRT]*/,
+                                                        double *__restrict__ wg_sums /*[nblk][2]*/) {
+  constexpr int CG = 256 / PX;
   __shared__ double sa[256], sb[256];
-  const int NRT = g.N_r * g.N_t;
-  const int rt = blockIdx.x * blockDim.x + threadIdx.x;
-  double a = 0.0, b = 0.0;
-  if (rt < NRT) {
-    double num = 0.0, den = 0.0;
-    for (int ch = 0; ch < nch; ch++) {
+  const int NRT = g.N_r * g.N_t, tid = threadIdx.x, px = tid % PX, cg = tid / PX;
+  const int rt = blockIdx.x * PX + px;
+  double num = 0.0, den = 0.0;
+  if (rt < NRT)
+    for (int ch = cg; ch < nch; ch += CG) {
       num += part[((size_t)ch * 2 + 0) * NRT + rt];
       den += part[((size_t)ch * 2 + 1) * NRT + rt];
     }
+  if (CG > 1) {
+    sa[tid] = num;
+    sb[tid] = den;
+    __syncthreads();
+    if (cg == 0)
+      for (int q = 1; q < CG; q++) {
+        num += sa[q * PX + px];
+        den += sb[q * PX + px];
+      }
+    __syncthreads();
+  }
+  double a = 0.0, b = 0.0;
+  if (rt < NRT && cg == 0) {
     numden[rt] = num;
     numden[NRT + rt] = den;
     a = (double)d[rt] + num / den;
     b = 1.0 / den;
   }
-  sa[threadIdx.x] = a;
-  sb[threadIdx.x] = b;
+  sa[tid] = a;
+  sb[tid] = b;
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      sa[threadIdx.x] += sa[threadIdx.x + s];
-      sb[threadIdx.x] += sb[threadIdx.x + s];
+  for (int s = PX / 2; s > 0; s >>= 1) {
+    if (tid < s) {
+      sa[tid] += sa[tid + s];
+      sb[tid] += sb[tid + s];
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     wg_sums[blockIdx.x * 2 + 0] = sa[0];
     wg_sums[blockIdx.x * 2 + 1] = sb[0];
   }
 }
 
-__global__ void k_offset_gamma(int nblk, const double *__restrict__ wg_sums, int zero_mean,
-                               double *__restrict__ gamma) {
+// d += step, e -= step.  Every workgroup forms gamma itself from the nblk partial sums (a
+// few KB out of L2, in the same order everywhere): a launch less than a kernel for it.
+__global__ void __launch_bounds__(256) k_offset_apply(XtGeom g, int chunk_views, int nblk,
+                                                      int zero_mean, const double *__restrict__ numden,
+                                                      const double *__restrict__ wg_sums,
+                                                      float *__restrict__ d, float *__restrict__ e) {
   __shared__ double sa[256], sb[256];
-  double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x) {
-    a += wg_sums[i * 2];
-    b += wg_sums[i * 2 + 1];
-  }
-  sa[threadIdx.x] = a;
-  sb[threadIdx.x] = b;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      sa[threadIdx.x] += sa[threadIdx.x + s];
-      sb[threadIdx.x] += sb[threadIdx.x + s];
+  double gamma = 0.0;
+  if (zero_mean) {
+    double a = 0.0, b = 0.0;
+    for (int i = threadIdx.x; i < nblk; i += 256) {
+      a += wg_sums[i * 2];
+      b += wg_sums[i * 2 + 1];
     }
+    sa[threadIdx.x] = a;
+    sb[threadIdx.x] = b;
     __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) {
+        sa[threadIdx.x] += sa[threadIdx.x + s];
+        sb[threadIdx.x] += sb[threadIdx.x + s];
+      }
+      __syncthreads();
+    }
+    gamma = sa[0] / sb[0];
   }
-  if (threadIdx.x == 0) *gamma = zero_mean ? sa[0] / sb[0] : 0.0;
-}
-
-__global__ void k_offset_apply(XtGeom g, int chunk_views, const double *__restrict__ numden,
-                               const double *__restrict__ gamma, float *__restrict__ d,
-                               float *__restrict__ e) {
   const int NRT = g.N_r * g.N_t;
   const int rt = blockIdx.x * blockDim.x + threadIdx.x;
   const int ch = blockIdx.y;
   if (rt >= NRT) return;
-  const float step = (float)((numden[rt] - *gamma) / numden[NRT + rt]);
+  const float step = (float)((numden[rt] - gamma) / numden[NRT + rt]);
   if (ch == 0) d[rt] = d[rt] + step;
   const int p0 = ch * chunk_views, p1 = min(g.N_p, p0 + chunk_views);
   const int r = rt / g.N_t, t = rt - (rt / g.N_t) * g.N_t;

@@ -325,7 +325,6 @@ struct xt_icd_state {
   uint64_t graph_opt_gen = 0;   // g_opt_gen when the graph was captured
   uint64_t lines_gen = 1;       // bumped when the line list or its NHICD shares change
   int64_t graph_launches = 0;   // voxel-update launches in the captured iteration
-  int off_nch = 1, off_chunk = 1, off_nblk = 1;
   // batched passes (k_icd_plane, k_icd_step): what they are launched with, for up
   // to pass_gx lines per step; the buffers are the state's, so every stream and
   // batch branch has its own
@@ -775,17 +774,46 @@ static int launch_order(xt_icd_state *s) {
   return XT_OK;
 }
 
-static int offset_update(xt_icd_state *s) {
+// The ring-offset update's split: view chunks so that pixels x chunks fill the chip, of 8
+// views (the loads a thread has in flight) or more, and the combine's workgroups.
+struct OffsetPlan {
+  int nch, chunk, nblk;
+  bool wide;  // 256 pixels a combine workgroup (few chunks)
+  OffsetPlan(int N_p, int NRT) {
+    nch = std::min({N_p, (262144 + NRT - 1) / NRT, (N_p + 7) / 8});
+    chunk = (N_p + nch - 1) / nch;
+    nch = (N_p + chunk - 1) / chunk;
+    wide = nch < 8;
+    nblk = wide ? (NRT + 255) / 256 : (NRT + 31) / 32;
+  }
+};
+
+static void offset_launch(hipStream_t st, const XtGeom &g, const OffsetPlan &o, int zero_mean,
+                          float *e, const float *w, float *d, double *part, double *numden,
+                          double *wg) {
+  const dim3 g2((g.N_r * g.N_t + 255) / 256, o.nch);
+  hipLaunchKernelGGL(k_offset_partial, g2, dim3(256), 0, st, g, e, w, o.chunk, part);
+  if (o.wide)
+    hipLaunchKernelGGL(k_offset_combine<256>, dim3(o.nblk), dim3(256), 0, st, g, o.nch, part, d,
+                       numden, wg);
+  else
+    hipLaunchKernelGGL(k_offset_combine<32>, dim3(o.nblk), dim3(256), 0, st, g, o.nch, part, d,
+                       numden, wg);
+  hipLaunchKernelGGL(k_offset_apply, g2, dim3(256), 0, st, g, o.chunk, o.nblk, zero_mean, numden, wg,
+                     d, e);
+}
+
+static int offset_alloc(xt_icd_state *s) {
   const int NRT = s->g.N_r * s->g.N_t;
-  dim3 g2((NRT + 255) / 256, s->off_nch);
-  hipLaunchKernelGGL(k_offset_partial, g2, dim3(256), 0, s->st, s->g, s->e, s->w, s->off_chunk,
-                     s->off_part);
-  hipLaunchKernelGGL(k_offset_combine, dim3(s->off_nblk), dim3(256), 0, s->st, s->g, s->off_nch,
-                     s->off_part, s->d, s->off_numden, s->off_wg);
-  hipLaunchKernelGGL(k_offset_gamma, dim3(1), dim3(256), 0, s->st, s->off_nblk, s->off_wg,
-                     s->zero_mean, s->scal);
-  hipLaunchKernelGGL(k_offset_apply, g2, dim3(256), 0, s->st, s->g, s->off_chunk, s->off_numden,
-                     s->scal, s->d, s->e);
+  const OffsetPlan o(s->g.N_p, NRT);
+  XT_TRY(dev_alloc(&s->off_part, (size_t)o.nch * 2 * NRT));
+  XT_TRY(dev_alloc(&s->off_numden, (size_t)2 * NRT));
+  return dev_alloc(&s->off_wg, (size_t)2 * o.nblk);
+}
+
+static int offset_update(xt_icd_state *s) {
+  offset_launch(s->st, s->g, OffsetPlan(s->g.N_p, s->g.N_r * s->g.N_t), s->zero_mean, s->e, s->w, s->d,
+                s->off_part, s->off_numden, s->off_wg);
   XT_HIP(hipGetLastError());
   return XT_OK;
 }
@@ -1349,20 +1377,7 @@ static int create_impl(Sinogram *S, ScannedObject *O, TomoInputs *T, xt_icd_stat
     return fail(rc);
   if (hipMemset(s->iter_dev, 0, sizeof(int)) != hipSuccess)
     return fail(set_err(XT_E_HIP, "iteration counter clear failed"));
-  // ring-offset scratch: view chunks so that N_r*N_t*chunks >= ~256k threads
-  {
-    const int NRT = g.N_r * g.N_t;
-    int nch = (262144 + NRT - 1) / NRT;
-    if (nch > g.N_p) nch = g.N_p;
-    if (nch < 1) nch = 1;
-    s->off_chunk = (g.N_p + nch - 1) / nch;
-    s->off_nch = (g.N_p + s->off_chunk - 1) / s->off_chunk;
-    s->off_nblk = (NRT + 255) / 256;
-    if ((rc = dev_alloc(&s->off_part, (size_t)s->off_nch * 2 * NRT)) ||
-        (rc = dev_alloc(&s->off_numden, (size_t)2 * NRT)) ||
-        (rc = dev_alloc(&s->off_wg, (size_t)2 * s->off_nblk)))
-      return fail(rc);
-  }
+  if ((rc = offset_alloc(s))) return fail(rc);
   if (src) {
     // y and w of a state over the same sinogram, already in the HBM layout
     const XtGeom &h = src->g;
@@ -2520,14 +2535,7 @@ extern "C" int xt_offset_update(Sinogram *S, TomoInputs *T, Real_t ***E) {
   const int NRT = S->N_r * S->N_t;
   XT_TRY(dev_alloc(&s->d, NRT));
   XT_HIP(real_to_dev(s->d, &S->ProjOffset[0][0], NRT));
-  int nch = (262144 + NRT - 1) / NRT;
-  if (nch > S->N_p) nch = S->N_p;
-  s->off_chunk = (S->N_p + nch - 1) / nch;
-  s->off_nch = (S->N_p + s->off_chunk - 1) / s->off_chunk;
-  s->off_nblk = (NRT + 255) / 256;
-  XT_TRY(dev_alloc(&s->off_part, (size_t)s->off_nch * 2 * NRT));
-  XT_TRY(dev_alloc(&s->off_numden, (size_t)2 * NRT));
-  XT_TRY(dev_alloc(&s->off_wg, (size_t)2 * s->off_nblk));
+  XT_TRY(offset_alloc(s));
   XT_TRY(dev_alloc(&s->scal, 8));
   XT_TRY(offset_update(s));
   XT_HIP(hipStreamSynchronize(s->st));
@@ -2569,22 +2577,17 @@ extern "C" int xt_offset_update_noalloc(int32_t N_p, int32_t N_r, int32_t N_t, f
     return set_err(XT_E_ARG, "empty sinogram %d x %d x %d", N_p, N_r, N_t);
   if ((size_t)N_p * N_r * N_t * sizeof(float) >= ((size_t)1 << 31))
     return set_err(XT_E_ARG, "sinogram of %d x %d x %d entries: at most 2^29 - 1", N_p, N_r, N_t);
-  // the view chunking of the allocating form (bit-identical results)
+  // the split of the allocating form (bit-identical results)
   const int NRT = N_r * N_t;
-  int nch = (262144 + NRT - 1) / NRT;
-  if (nch > N_p) nch = N_p;
-  const int chunk = (N_p + nch - 1) / nch;
-  nch = (N_p + chunk - 1) / chunk;
-  const int nblk = (NRT + 255) / 256;
-  const size_t need = (size_t)2 * nch * NRT + (size_t)2 * NRT + (size_t)2 * nblk + 8;
+  const OffsetPlan o(N_p, NRT);
+  const size_t need = (size_t)2 * o.nch * NRT + (size_t)2 * NRT + (size_t)2 * o.nblk + 8;
   if (need > XT_NOALLOC_SCRATCH_DOUBLES)
     return set_err(XT_E_ARG, "%d x %d detector pixels need %zu B of offset scratch; the "
                    "allocation-free form holds %zu B (at most about 131072 pixels)", N_r, N_t,
                    need * sizeof(double), (size_t)XT_NOALLOC_SCRATCH_DOUBLES * sizeof(double));
   double *base = nullptr;
   XT_TRY(noalloc_scratch(&base));
-  double *part = base, *numden = part + (size_t)2 * nch * NRT, *wg = numden + (size_t)2 * NRT,
-         *gamma = wg + (size_t)2 * nblk;
+  double *part = base, *numden = part + (size_t)2 * o.nch * NRT, *wg = numden + (size_t)2 * NRT;
   XtGeom g;
   memset(&g, 0, sizeof g);
   g.N_p = N_p;
@@ -2592,12 +2595,7 @@ extern "C" int xt_offset_update_noalloc(int32_t N_p, int32_t N_r, int32_t N_t, f
   g.N_t = N_t;
   g.T = zinger_T;
   g.delta = zinger_delta;
-  const dim3 g2((NRT + 255) / 256, nch);
-  hipLaunchKernelGGL(k_offset_partial, g2, dim3(256), 0, 0, g, E, W, chunk, part);
-  hipLaunchKernelGGL(k_offset_combine, dim3(nblk), dim3(256), 0, 0, g, nch, part, ProjOffset,
-                     numden, wg);
-  hipLaunchKernelGGL(k_offset_gamma, dim3(1), dim3(256), 0, 0, nblk, wg, zero_mean ? 1 : 0, gamma);
-  hipLaunchKernelGGL(k_offset_apply, g2, dim3(256), 0, 0, g, chunk, numden, gamma, ProjOffset, E);
+  offset_launch(0, g, o, zero_mean ? 1 : 0, E, W, ProjOffset, part, numden, wg);
   XT_HIP(hipGetLastError());
   XT_HIP(hipStreamSynchronize(0));
   return XT_OK;
