@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from conftest import SMALL, TINY
-from test_gpu_parity import NZ32, NZ64, _pair, _print_case
+from test_gpu_parity import NZ32, NZ64, WIDE3, WIDE6, _pair, _print_case
 from timbir_python_amd import xt_abi, xt_hip
 
 pytestmark = pytest.mark.gpu
@@ -33,14 +33,18 @@ def _slices(O, T, parity):
     return [z for z in zs if z % 2 == 0] + [z for z in zs if z % 2]
 
 
-@pytest.mark.parametrize("cfg", [TINY, SMALL, NZ32, NZ64, ODD5, LAST4, WIDE65], ids=lambda c: c.name)
+# SMALL without its table and the voxels wider than two bins: columns computed in the pass
+@pytest.mark.parametrize("cfg,atable", [(c, 1) for c in (TINY, SMALL, NZ32, NZ64, ODD5, LAST4, WIDE65,
+                                                          WIDE3, WIDE6)] + [(SMALL, 0)],
+                         ids=lambda c: getattr(c, "name", f"atable{c}"))
 @pytest.mark.parametrize("lines", [1, 20])
 @pytest.mark.parametrize("parity,Iter", [(0, 1), (1, 2)])
-def test_batched_pass_per_voxel(parity, Iter, lines, cfg, scan_root, oracle32):
+def test_batched_pass_per_voxel(parity, Iter, lines, cfg, atable, scan_root, oracle32):
     _print_case(f"batched pass lines={lines} parity={parity} Iter={Iter}", cfg)
     path, info, eng, (S, O, T) = _pair(cfg, scan_root, oracle32)
     xt_hip.set_option(xt_hip.OPT_PASS, 2)
     xt_hip.set_option(xt_hip.OPT_LINES, lines)
+    xt_hip.set_option(xt_hip.OPT_ATABLE, atable)
     try:
         vol = (0.7 * info["phantom"]).astype(np.float32)
         vol[:, :, :4, :] = 0  # zero rows: zero-skipping paths
@@ -89,5 +93,6 @@ def test_batched_pass_per_voxel(parity, Iter, lines, cfg, scan_root, oracle32):
     finally:
         xt_hip.set_option(xt_hip.OPT_PASS, 0)
         xt_hip.set_option(xt_hip.OPT_LINES, 0)
+        xt_hip.set_option(xt_hip.OPT_ATABLE, 1)
         eng.close()
         oracle32.free(S, O, T)

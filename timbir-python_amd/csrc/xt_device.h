@@ -1132,17 +1132,22 @@ __global__ void __launch_bounds__(NT) k_icd_lines(XtGeom g, XtIcdBuffers B, XtIc
 // (line, entry).  k_icd_step reduces the theta partials and takes the surrogate
 // step of every voxel of the step's lines, the 26 neighbours of a voxel spread
 // over its R threads.
+#define XT_PASS_NG 4  // 4-bin groups that hold a column of up to XT_MAXA_WIDE entries
+
 struct XtPass {
   int gx;        // lines per step and frame
   int S;         // slices of a parity (LDS slots before padding to ZC)
   int nvc, vch;  // view chunks of a frame, views per chunk
   int nzc;       // slot chunks of ZC
   const int *order;    // [N_time][2][n_lines]: the iteration's line order (k_icd_order)
-  float4 *ga;          // [2][N_time][max_views][gx] column values of a step's lines, x delta_t,
-  int *gb;             // and their first bins: even and odd steps
+  int ng;              // 4-bin groups of a column: 1 (from the table) or XT_PASS_NG (computed)
+  float4 *ga;          // [2][N_time][max_views][ng][gx] column values of a step's lines, x
+  int *gb;             // delta_t, and their first bins (ng > 1: plus their entries << 20):
+                       // even and odd steps
+  int *gcnt;           // ng > 1: [2][N_time][gx] footprint entries of the step's lines
   float2 *part;        // [N_time][nvc][gx][S] theta1, theta2 partials
   float *dlt;          // [N_time][gx][S] the step's changes
-  const int *cnt_col;  // [N_time][N_y*N_x] footprint entries of a line's column
+  const int *cnt_col;  // ng == 1: [N_time][N_y*N_x] footprint entries of a line's column
   double *st_wg;       // [workgroups of k_icd_step][4] statistics of the iteration
   uint8_t zmap[2][64];  // slice of the k-th slot of a parity, 255 past its last
   uint8_t zblk[2][64];  // its z-block
@@ -1247,10 +1252,65 @@ __device__ __forceinline__ void xt_gather_tile(const XtGeom &g, const XtIcdBuffe
   }
 }
 
+// The same with columns computed on the spot (voxels wider than two bins, or no table):
+// 16 lines x 16 views a workgroup, a column a thread, its entries moved to the front.
+// 256 lines x 1024 views of 14 candidate bins take about as long as a table read of them.
+template <int MA>
+__device__ __forceinline__ void xt_gather_columns(const XtGeom &g, const XtIcdBuffers &B,
+                                                  const XtPass &P, const XtPassList &R, int step,
+                                                  int f, int tile) {
+  const int tid = threadIdx.x, nvt = (g.max_views + 15) / 16;
+  const int j = (tile / nvt) * 16 + (tid & 15), p = (tile % nvt) * 16 + (tid >> 4);
+  const int c = xt_pass_line(R, P.gx, step, j);
+  int n = 0;
+  if (j < P.gx && p < g.max_views) {
+    float v[4 * XT_PASS_NG];
+#pragma unroll
+    for (int b = 0; b < 4 * XT_PASS_NG; b++) v[b] = 0.f;
+    int first = 0;
+    if (c >= 0 && p < B.proj_num[f]) {
+      const int vw = B.views[(size_t)f * g.max_views + p];
+      const int yy = c / g.N_x, xx = c - yy * g.N_x;
+      float vals[MA];
+      xt_amatrix_column(g, B.Hr + (size_t)vw * XT_HR_STRIDE, B.cosv[vw], B.sinv[vw], yy, xx, &first,
+                        vals);
+      int b0 = 0, last = -1;
+#pragma unroll
+      for (int b = MA - 1; b >= 0; b--) {
+        v[b] = vals[b] * g.delta_t;
+        if (vals[b] > 0.f) {
+          b0 = b;
+          last = last < 0 ? b : last;
+          n++;
+        }
+      }
+#pragma unroll
+      for (int sh = 1; sh < 16; sh <<= 1)  // v[i] = v[i + b0], a bit of b0 at a time
+#pragma unroll
+        for (int b = 0; b < MA; b++)
+          v[b] = (b0 & sh) ? (b + sh < MA ? v[b + sh] : 0.f) : v[b];
+      first += b0;
+      const int len = last < 0 ? 0 : last - b0 + 1;
+      first = len ? first + (len << 20) : 0;
+    }
+    const size_t row = ((size_t)(step & 1) * g.N_time + f) * g.max_views + p;
+#pragma unroll
+    for (int q = 0; q < XT_PASS_NG; q++)
+      P.ga[(row * XT_PASS_NG + q) * P.gx + j] =
+          make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+    P.gb[row * P.gx + j] = first;
+  }
+  // entries of a line over the tile's views: 4 views of a wave, then one add a line and wave
+  n += __shfl_xor(n, 16);
+  n += __shfl_xor(n, 32);
+  if ((tid & 63) < 16 && j < P.gx && n)
+    atomicAdd(&P.gcnt[((size_t)(step & 1) * g.N_time + f) * P.gx + j], n);
+}
+
 // One step over the views: grid (view chunks x slot chunks, frames), threads for ZC
 // slots and LG lines at a time, I lines per thread (gx <= I * LG).
 // Applies the changes of step - 1 and sums theta for step.
-template <int ZC, int LG, int I>
+template <int ZC, int LG, int I, int NG>
 __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers B,
                                                                     XtIcdLaunch L, XtPass P,
                                                                     int step) {
@@ -1276,11 +1336,13 @@ __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers 
   }
   const int nr = (g.N_r + LG - 1) / LG;  // bins of a row per thread
   extern __shared__ float4 smem4[];
-  float4 *av = smem4;              // [I * LG] a step's column values of the view, 0 past gx
-  int *ab = (int *)(av + I * LG);  // [I * LG] its first LDS row
-  // [nr * LG + 3][ZC]: e as doubles while the changes are applied (an LDS atomic add
+  constexpr int LN = I * LG;
+  float4 *av = smem4;              // [NG][LN] a step's column values of the view, 0 past gx
+  int *ab = (int *)(av + NG * LN);  // [LN] its first LDS row
+  int *mx = ab + LN;               // [4] NG > 1: entries of the longest column, prev and cur
+  // [nr * LG + 4 NG - 1][ZC]: e as doubles while the changes are applied (an LDS atomic add
   // takes 14 clocks a wave in FP64 and 194 in FP32 on gfx950), then (ws, e ws); 0 past N_r
-  float2 *pl = (float2 *)(ab + I * LG);
+  float2 *pl = (float2 *)(mx + (NG > 1 ? 4 : 0));
   double *pd = (double *)pl;
   const int slot = zc * ZC + k;
   const bool on = slot < P.S && P.zmap[par][slot] != 255;
@@ -1306,14 +1368,23 @@ __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers 
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       const int j = tid + s * NT;
-      if (j < I * LG) {
-        av[j] = j < P.gx ? P.ga[row + j] : make_float4(0.f, 0.f, 0.f, 0.f);
-        ab[j] = j < P.gx ? P.gb[row + j] * ZC : 0;
+      if (j < LN) {
+#pragma unroll
+        for (int c = 0; c < NG; c++)
+          av[c * LN + j] =
+              j < P.gx ? P.ga[row * NG + (size_t)c * P.gx + j] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const int b = j < P.gx ? P.gb[row + j] : 0;
+        ab[j] = (NG > 1 ? b & 0xFFFFF : b) * ZC;
+        if (NG > 1) atomicMax(&mx[st == step], b >> 20);
       }
     }
   };
-  // a column may reach past the last bin with zero entries: three spare rows
-  if (tid < 3 * ZC) pl[nr * LG * ZC + tid] = make_float2(0.f, 0.f);
+  // a column may reach past the last bin with zero entries: spare rows
+  for (int q = tid; q < (4 * NG - 1) * ZC; q += NT) pl[nr * LG * ZC + q] = make_float2(0.f, 0.f);
+  if (NG > 1) {
+    if (tid < 2) mx[tid] = 0;
+    __syncthreads();
+  }
   const float T2 = g.T * g.T, Td = g.T * g.delta;
   // a view's rows of e and w through buffer descriptors that end with its last bin: an
   // offset past it, or a slot that is off, reads 0 and drops the store
@@ -1349,16 +1420,22 @@ __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers 
       }
       stage(step - 1, p);
       __syncthreads();
+      const int nc = NG > 1 ? mx[0] : 4;
+      if (NG > 1 && tid == 0) mx[1] = 0;
       // e -= A * delta
 #pragma unroll
       for (int i = 0; i < I; i++) {
         if (dl[i] != 0.f) {
-          const float4 a = av[lg + i * LG];
           double *q = pd + ab[lg + i * LG] + k;
-          atomicAdd(q, (double)-(a.x * dl[i]));
-          atomicAdd(q + ZC, (double)-(a.y * dl[i]));
-          atomicAdd(q + 2 * ZC, (double)-(a.z * dl[i]));
-          atomicAdd(q + 3 * ZC, (double)-(a.w * dl[i]));
+#pragma unroll
+          for (int c = 0; c < NG; c++)
+            if (4 * c < nc) {
+              const float4 a = av[c * LN + lg + i * LG];
+              atomicAdd(q + 4 * c * ZC, (double)-(a.x * dl[i]));
+              atomicAdd(q + (4 * c + 1) * ZC, (double)-(a.y * dl[i]));
+              atomicAdd(q + (4 * c + 2) * ZC, (double)-(a.z * dl[i]));
+              atomicAdd(q + (4 * c + 3) * ZC, (double)-(a.w * dl[i]));
+            }
         }
         __builtin_amdgcn_sched_barrier(0);  // in the compiler's order the lines spill
       }
@@ -1391,13 +1468,20 @@ __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers 
     if (cur) {
       stage(step, p);
       __syncthreads();
+      const int nc = NG > 1 ? mx[1] : 4;
+      if (NG > 1 && tid == 0) mx[0] = 0;
 #pragma unroll
       for (int i = 0; i < I; i++) {
-        const float4 a = av[lg + i * LG];
-        const float2 *q = pl + ab[lg + i * LG] + k;
-        const float2 u0 = q[0], u1 = q[ZC], u2 = q[2 * ZC], u3 = q[3 * ZC];
-        t2[i] += a.x * (a.x * u0.x) + a.y * (a.y * u1.x) + a.z * (a.z * u2.x) + a.w * (a.w * u3.x);
-        t1[i] -= a.x * u0.y + a.y * u1.y + a.z * u2.y + a.w * u3.y;
+        const float2 *q0 = pl + ab[lg + i * LG] + k;
+#pragma unroll
+        for (int c = 0; c < NG; c++)
+          if (4 * c < nc) {
+            const float4 a = av[c * LN + lg + i * LG];
+            const float2 *q = q0 + 4 * c * ZC;
+            const float2 u0 = q[0], u1 = q[ZC], u2 = q[2 * ZC], u3 = q[3 * ZC];
+            t2[i] += a.x * (a.x * u0.x) + a.y * (a.y * u1.x) + a.z * (a.z * u2.x) + a.w * (a.w * u3.x);
+            t1[i] -= a.x * u0.y + a.y * u1.y + a.z * u2.y + a.w * u3.y;
+          }
         if (i & 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -1429,10 +1513,15 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
   const int par = L.mode == 3 ? L.half : ((L.half ^ f) & 1);
   const XtPassList Q = xt_pass_list(g, B, L, P, f, par);
   constexpr int kTile = 64 * 17 * (sizeof(float4) + sizeof(int));
-  constexpr int kStep = 32 + 256 * sizeof(float2) + LW * (66 + 64 + 1) * sizeof(float);
+  constexpr int kStep = 32 + 256 * sizeof(float2) + LW * (66 + 64 + 2) * sizeof(float);
   __shared__ __align__(16) char smem[kTile > kStep ? kTile : kStep];
   if ((int)blockIdx.x >= nwg) {
-    if (step + 1 < Q.steps) xt_gather_tile(g, B, P, Q, step + 1, f, (int)blockIdx.x - nwg, smem);
+    if (step + 1 < Q.steps) {
+      const int tile = (int)blockIdx.x - nwg;
+      if (P.ng == 1) xt_gather_tile(g, B, P, Q, step + 1, f, tile, smem);
+      else if (g.wide) xt_gather_columns<XT_MAXA_WIDE>(g, B, P, Q, step + 1, f, tile);
+      else xt_gather_columns<XT_MAXA>(g, B, P, Q, step + 1, f, tile);
+    }
     return;
   }
   if (step >= Q.steps) return;
@@ -1440,7 +1529,7 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
   float2 *red = (float2 *)(st + 4);         // [256]
   float(*xs)[66] = (float(*)[66])(red + 256);  // [LW]
   float(*magb)[64] = (float(*)[64])(xs + LW);  // [LW]
-  int *cl = (int *)(magb + LW);             // [LW] the workgroup's lines
+  int *cl = (int *)(magb + LW);             // [2 LW] the workgroup's lines, their entries
   const size_t NYX = (size_t)g.N_y * g.N_x;
   const int iter = *B.iter, nz = g.N_z;
   // the voxel of this thread: pair = (line l, slot kk), its share r of the neighbours;
@@ -1457,7 +1546,14 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
   const int yy = c >= 0 ? c / g.N_x : 0, xx = c >= 0 ? c - yy * g.N_x : 0;
   if (tid < 4) st[tid] = 0.0;
   constexpr int TL = SP * R;  // threads of a line
-  if (tid % TL == 0) cl[l] = c;
+  if (tid % TL == 0) {
+    cl[l] = c;
+    if (P.ng > 1 && j < P.gx) {  // taken, and zero for the step after next
+      int *n = &P.gcnt[((size_t)(step & 1) * g.N_time + f) * P.gx + j];
+      cl[LW + l] = *n;
+      *n = 0;
+    }
+  }
   for (int zz = tid % TL; zz < 64; zz += TL) {
     xs[l][zz] = (c >= 0 && zz < nz)
                     ? __hip_atomic_load(&B.x[((size_t)f * NYX + c) * nz + zz], __ATOMIC_RELAXED,
@@ -1547,7 +1643,7 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
       atomicAdd(&magb[l][P.zblk[par][kk]], fabsf(change));
       if (L.count_stats) atomicAdd(&st[0], (double)fabsf(nv2));
       atomicAdd(&st[1], 1.0);
-      atomicAdd(&st[2], (double)P.cnt_col[(size_t)f * NYX + c]);
+      atomicAdd(&st[2], (double)(P.ng == 1 ? P.cnt_col[(size_t)f * NYX + c] : cl[LW + l]));
     }
     __syncthreads();
   }

@@ -335,7 +335,7 @@ struct xt_icd_state {
   int *order = nullptr, *cnt_col = nullptr;
   float2 *pass_part = nullptr;
   float4 *pass_ga = nullptr;
-  int *pass_gb = nullptr;
+  int *pass_gb = nullptr, *pass_cnt = nullptr;
   float *pass_dlt = nullptr;
   double *st_wg = nullptr;
   int st_n = 0;
@@ -362,7 +362,7 @@ static void free_state(xt_icd_state *s) {
                   s->red_wg,   s->scal,       s->off_part, s->off_numden, s->off_wg,
                   s->at_vals,  s->at_first,   s->iter_dev, s->pc_tmp, s->vmask, s->vsc_st,
                   s->vsc_hist, s->order, s->cnt_col,
-                  s->pass_part, s->pass_dlt, s->st_wg, s->pass_ga, s->pass_gb};
+                  s->pass_part, s->pass_dlt, s->st_wg, s->pass_ga, s->pass_gb, s->pass_cnt};
   if (s->graph_exec) (void)hipGraphExecDestroy(s->graph_exec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   for (void *b : bufs)
@@ -504,28 +504,35 @@ static int pass_rows(int gx) {  // lines per thread, the variant's
   return I <= 1 ? 1 : I <= 2 ? 2 : I <= 4 ? 4 : I <= 8 ? 8 : 16;
 }
 
-static size_t pass_lds(const XtGeom &g, int zc, int gx) {
-  return (size_t)pass_rows(gx) * kPassRow * (sizeof(float4) + sizeof(int)) +
-         (size_t)((g.N_r + kPassRow - 1) / kPassRow * kPassRow + 3) * zc * sizeof(float2);
+static size_t pass_lds(const XtGeom &g, int zc, int ng, int gx) {
+  return (size_t)pass_rows(gx) * kPassRow * (ng * sizeof(float4) + sizeof(int)) +
+         (ng > 1 ? 16 : 0) +
+         (size_t)((g.N_r + kPassRow - 1) / kPassRow * kPassRow + 4 * ng - 1) * zc * sizeof(float2);
 }
 
 // f(kernel, threads) on the k_icd_plane instantiation for zc slots and gx lines
-template <int ZC, typename F>
+template <int ZC, int NG, typename F>
 static void plane_pick(int gx, F f) {
   constexpr int LG = kPassRow;
   const int I = pass_rows(gx);
-  if (I <= 1) f(k_icd_plane<ZC, LG, 1>, ZC * LG);
-  else if (I <= 2) f(k_icd_plane<ZC, LG, 2>, ZC * LG);
-  else if (I <= 4) f(k_icd_plane<ZC, LG, 4>, ZC * LG);
-  else if (I <= 8) f(k_icd_plane<ZC, LG, 8>, ZC * LG);
-  else f(k_icd_plane<ZC, LG, 16>, ZC * LG);
+  if (I <= 1) f(k_icd_plane<ZC, LG, 1, NG>, ZC * LG);
+  else if (I <= 2) f(k_icd_plane<ZC, LG, 2, NG>, ZC * LG);
+  else if (I <= 4) f(k_icd_plane<ZC, LG, 4, NG>, ZC * LG);
+  else if (I <= 8) f(k_icd_plane<ZC, LG, 8, NG>, ZC * LG);
+  else f(k_icd_plane<ZC, LG, 16, NG>, ZC * LG);
 }
 
 template <typename F>
-static void plane_pick(int zc, int gx, F f) {
-  if (zc == 4) plane_pick<4>(gx, f);
-  else if (zc == 8) plane_pick<8>(gx, f);
-  else plane_pick<16>(gx, f);
+static void plane_pick(int zc, int ng, int gx, F f) {
+  if (ng == 1) {
+    if (zc == 4) plane_pick<4, 1>(gx, f);
+    else if (zc == 8) plane_pick<8, 1>(gx, f);
+    else plane_pick<16, 1>(gx, f);
+  } else {
+    if (zc == 4) plane_pick<4, XT_PASS_NG>(gx, f);
+    else if (zc == 8) plane_pick<8, XT_PASS_NG>(gx, f);
+    else plane_pick<16, XT_PASS_NG>(gx, f);
+  }
 }
 
 // slots of a line and threads per voxel of k_icd_step: 16 threads share a voxel's
@@ -547,8 +554,9 @@ static void step_go(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B, cons
                     const XtPass &P, int step, bool gather) {
   constexpr int lw = 256 / (SP * R);
   const int nwg = step < 0 ? 0 : (P.gx + lw - 1) / lw;
-  const int ng = gather ? ((P.gx + 15) / 16) * ((g.max_views + 63) / 64) : 0;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R>), dim3(nwg + ng, g.N_time), dim3(256), 0, st, g,
+  const int tv = P.ng == 1 ? 64 : 16;  // views of a gather workgroup
+  const int tiles = gather ? ((P.gx + 15) / 16) * ((g.max_views + tv - 1) / tv) : 0;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R>), dim3(nwg + tiles, g.N_time), dim3(256), 0, st, g,
                      B, L, P, step, nwg);
 }
 
@@ -583,7 +591,7 @@ static int pass_alloc(T **p, size_t n) {
 static int plan_pass(xt_icd_state *s, int gx) {
   const XtGeom &g = s->g;
   s->pass_ok = false;
-  if (!s->at_vals || g.wide || g.pc || g.zo != 1 || gx < 1 || gx > 1024 ||
+  if (g.pc || g.zo != 1 || gx < 1 || gx > 1024 ||
       s->NYX > ((size_t)1 << 22))
     return XT_OK;
   XtPass &P = s->pass;
@@ -607,11 +615,12 @@ static int plan_pass(xt_icd_state *s, int gx) {
   // as many slots of a bin together as there are (up to 16: a wave's LDS accesses then
   // fall into 4 runs of 128 bytes instead of 16 of 32; 512^2 x 32, two iterations: 247 ms
   // with 16 slots, 261 with 8, 345 with 4), while the rows fit the LDS
+  P.ng = s->at_vals ? 1 : XT_PASS_NG;
   int zc = P.S <= 4 ? 4 : P.S <= 8 ? 8 : 16;
   int lds_max = 0;
   (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->dev);
-  while (zc > 4 && pass_lds(g, zc, gx) > (size_t)lds_max) zc /= 2;
-  const size_t lds = pass_lds(g, zc, gx);
+  while (zc > 4 && pass_lds(g, zc, P.ng, gx) > (size_t)lds_max) zc /= 2;
+  const size_t lds = pass_lds(g, zc, P.ng, gx);
   if (lds > (size_t)lds_max) return XT_OK;
   s->pass_zc = zc;
   P.nzc = (P.S + zc - 1) / zc;
@@ -626,7 +635,7 @@ static int plan_pass(xt_icd_state *s, int gx) {
   if (lds > 64 * 1024) {
     hipError_t e = hipSuccess;
     for (int n = kPassRow; n <= 1024; n *= 2)  // every lines-per-thread variant
-      plane_pick(zc, n, [&](auto k, int) {
+      plane_pick(zc, P.ng, n, [&](auto k, int) {
         if (e == hipSuccess)
           e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       });
@@ -638,11 +647,13 @@ static int plan_pass(xt_icd_state *s, int gx) {
   const size_t fg = (size_t)g.N_time * gx, fv = (size_t)2 * fg * g.max_views;
   // without the memory for them the line kernel serves
   if (pass_alloc(&s->pass_part, fg * P.nvc * P.S) || pass_alloc(&s->pass_dlt, fg * P.S) ||
-      pass_alloc(&s->pass_ga, fv) || pass_alloc(&s->pass_gb, fv) ||
+      pass_alloc(&s->pass_ga, fv * P.ng) || pass_alloc(&s->pass_gb, fv) ||
+      pass_alloc(&s->pass_cnt, 2 * fg) ||
       pass_alloc(&s->st_wg, (size_t)s->st_n * 4) ||
       (!s->order && pass_alloc(&s->order, (size_t)g.N_time * 2 * s->NYX)))
     return XT_OK;
-  if (!s->cnt_col) {
+  XT_HIP(hipMemsetAsync(s->pass_cnt, 0, 2 * fg * sizeof(int), s->st));
+  if (P.ng == 1 && !s->cnt_col) {
     if (pass_alloc(&s->cnt_col, (size_t)g.N_time * s->NYX)) return XT_OK;
     hipLaunchKernelGGL(k_col_count, dim3((unsigned)((s->NYX + 3) / 4), g.N_time), dim3(256), 0, s->st,
                        g, s->proj_num, s->at_vals, s->cnt_col);
@@ -653,6 +664,7 @@ static int plan_pass(xt_icd_state *s, int gx) {
   P.dlt = s->pass_dlt;
   P.ga = s->pass_ga;
   P.gb = s->pass_gb;
+  P.gcnt = s->pass_cnt;
   P.cnt_col = s->cnt_col;
   P.st_wg = s->st_wg;
   s->pass_ok = true;
@@ -706,9 +718,9 @@ static int launch_pass(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
   const int steps = pass_steps(s, L.mode, L.sub_iter, L.K, gx);
   if (steps > 0) step_launch(s->st, s->g, B, L, P, -1, true);
   for (int t = 0; t <= steps && steps > 0; t++) {
-    plane_pick(s->pass_zc, gx, [&](auto k, int nt) {
+    plane_pick(s->pass_zc, P.ng, gx, [&](auto k, int nt) {
       hipLaunchKernelGGL(k, dim3(P.nvc * P.nzc, s->g.N_time), dim3(nt),
-                         pass_lds(s->g, s->pass_zc, gx), s->st, s->g, B, L, P, t);
+                         pass_lds(s->g, s->pass_zc, P.ng, gx), s->st, s->g, B, L, P, t);
     });
     if (t < steps) step_launch(s->st, s->g, B, L, P, t, t + 1 < steps);
   }
