@@ -1504,7 +1504,8 @@ __global__ void __launch_bounds__(ZC *LG, 4) k_icd_plane(XtGeom g, XtIcdBuffers 
 // launch on, and lines of one step read each other's old or new x, as lines in flight
 // do.  The workgroups past the first nwg gather the next step's columns; step -1 does that
 // alone.
-template <int SP, int R>
+// MA: candidate bins of a computed column, 0 with the table.
+template <int SP, int R, int MA>
 __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIcdLaunch L, XtPass P,
                                                   int step, int nwg) {
   constexpr int PN = 256 / R, LW = PN / SP;  // (line, slot) pairs and lines of the workgroup
@@ -1518,9 +1519,8 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
   if ((int)blockIdx.x >= nwg) {
     if (step + 1 < Q.steps) {
       const int tile = (int)blockIdx.x - nwg;
-      if (P.ng == 1) xt_gather_tile(g, B, P, Q, step + 1, f, tile, smem);
-      else if (g.wide) xt_gather_columns<XT_MAXA_WIDE>(g, B, P, Q, step + 1, f, tile);
-      else xt_gather_columns<XT_MAXA>(g, B, P, Q, step + 1, f, tile);
+      if constexpr (MA == 0) xt_gather_tile(g, B, P, Q, step + 1, f, tile, smem);
+      else xt_gather_columns<MA>(g, B, P, Q, step + 1, f, tile);
     }
     return;
   }
@@ -1548,7 +1548,7 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
   constexpr int TL = SP * R;  // threads of a line
   if (tid % TL == 0) {
     cl[l] = c;
-    if (P.ng > 1 && j < P.gx) {  // taken, and zero for the step after next
+    if (MA != 0 && j < P.gx) {  // taken, and zero for the step after next
       int *n = &P.gcnt[((size_t)(step & 1) * g.N_time + f) * P.gx + j];
       cl[LW + l] = *n;
       *n = 0;
@@ -1643,7 +1643,7 @@ __global__ void __launch_bounds__(256) k_icd_step(XtGeom g, XtIcdBuffers B, XtIc
       atomicAdd(&magb[l][P.zblk[par][kk]], fabsf(change));
       if (L.count_stats) atomicAdd(&st[0], (double)fabsf(nv2));
       atomicAdd(&st[1], 1.0);
-      atomicAdd(&st[2], (double)(P.ng == 1 ? P.cnt_col[(size_t)f * NYX + c] : cl[LW + l]));
+      atomicAdd(&st[2], (double)(MA == 0 ? P.cnt_col[(size_t)f * NYX + c] : cl[LW + l]));
     }
     __syncthreads();
   }

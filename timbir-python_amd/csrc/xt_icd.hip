@@ -556,8 +556,16 @@ static void step_go(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B, cons
   const int nwg = step < 0 ? 0 : (P.gx + lw - 1) / lw;
   const int tv = P.ng == 1 ? 64 : 16;  // views of a gather workgroup
   const int tiles = gather ? ((P.gx + 15) / 16) * ((g.max_views + tv - 1) / tv) : 0;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R>), dim3(nwg + tiles, g.N_time), dim3(256), 0, st, g,
-                     B, L, P, step, nwg);
+  const dim3 grid(nwg + tiles, g.N_time);
+  if (P.ng == 1)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R, 0>), grid, dim3(256), 0, st, g, B, L, P, step,
+                       nwg);
+  else if (!g.wide)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R, XT_MAXA>), grid, dim3(256), 0, st, g, B, L, P,
+                       step, nwg);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_step<SP, R, XT_MAXA_WIDE>), grid, dim3(256), 0, st, g, B,
+                       L, P, step, nwg);
 }
 
 static void step_launch(hipStream_t st, const XtGeom &g, const XtIcdBuffers &B, const XtIcdLaunch &L,
