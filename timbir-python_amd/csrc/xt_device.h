@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define XT_MAXA 6          // max detector bins of one A column (2*delta_xy/delta_r + 2)
 #define XT_MAXA_WIDE 14    // the same for voxels up to 6 detector bins wide (coarse stages)
 #define XT_NBINS 64        // DETECTOR_RESPONSE_BINS
@@ -2385,19 +2387,32 @@ __device__ __forceinline__ float xt_pc_entry(const float (&vals)[XT_MAXA], int r
 // over the view groups in LDS and over the slice's three rows by the slice's own
 // thread, which takes the qGGMRF step; then e -= A * delta and a wait before the
 // next phase reads e.  Lines, the z-block parity and NHICD lists as k_icd_lines.
-template <int ZL>
-__global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, XtIcdLaunch L) {
-  constexpr int NT = 256, RL = ZL, G = NT / RL;  // row lanes of a view group, view groups
+// Few lines are in flight (the footprints couple more than absorption ones), so a visit's
+// latency is what bounds it: 16 waves a line while that leaves a CU per line, the e and w
+// of a view's footprint row loaded together (6 bins, two views at a time; bins 6 and 7
+// only on a line that has them) by branch-free buffer loads, and a slice's prior spread
+// over 32 lanes.  144 lines of 192^2 x 16 with 240 views, a launch over the whole plane:
+// 5.75 ms with 4 waves, a load after the other and the prior by one thread; 2.45 ms with
+// 16 waves and the loads together; 1.68 ms with the prior spread and 6 bins.  Three views
+// at a time spill registers (+15%).
+template <int ZL, int NT>
+__global__ void __launch_bounds__(NT) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, XtIcdLaunch L) {
+  constexpr int RL = ZL, G = NT / RL;  // row lanes of a view group, view groups
+  constexpr bool BUF = NT > 256;          // the sinogram fits a buffer's 2 GiB
+  constexpr uint32_t OOB = 0x80000000u;   // buffer offset that reads 0
   extern __shared__ float4 smem4[];
   float4 *a_v4 = smem4;                           // [max_views] bins 0..3 (x delta_t)
   float2 *a_v2 = (float2 *)(a_v4 + g.max_views);  // [max_views] bins 4..5
   int *a_first = (int *)(a_v2 + g.max_views);     // [max_views] first candidate bin
-  float *red1 = (float *)(a_first + g.max_views);  // [G][RL]
-  float *red2 = red1 + NT;                         // [G][RL]
-  float *xn = red2 + NT;                           // [11][ZL]
+  float *red1 = (float *)(a_first + g.max_views);  // [waves][RL]
+  float *red2 = red1 + NT / 64 * RL;               // [waves][RL]
+  float *xn = red2 + NT / 64 * RL;                 // [11][ZL]
   float *delta = xn + 11 * ZL;                     // [ZL]
-  float *magb = delta + ZL;                        // [64]
-  __shared__ int s_cnt;
+  float *ps1 = delta + ZL;                         // [ZL] prior's sums of the phase's slices
+  float *ps2 = ps1 + ZL;                           // [ZL]
+  float *magb = ps2 + ZL;                          // [64]
+  int *a_view = (int *)(magb + 64);                // [max_views] views, the wide group only
+  __shared__ int s_cnt, s_far;
   const int tid = threadIdx.x, grp = tid / RL, lt = tid % RL;
   const int f = blockIdx.y;
   const int nv = B.proj_num[f];
@@ -2436,6 +2451,11 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
   // the Laplacian weights of the lane's row for each row offset dt = -1, 0, 1
   // come from column 1 - dt of Lap_Kernel
   const int nph = L.zorder ? (g.N_z > 3 ? g.N_z : 3) : 3;
+  const uint32_t sino_bytes =
+      BUF ? (uint32_t)((size_t)g.N_p * g.N_r * g.N_t * sizeof(float)) : 0u;
+  const __amdgpu_buffer_rsrc_t rs_e = __builtin_amdgcn_make_buffer_rsrc(B.e, 0, sino_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_w =
+      __builtin_amdgcn_make_buffer_rsrc((void *)B.w, 0, sino_bytes, 0x00020000);
   float vox_mag = 0.f;
   double n_upd = 0.0, n_foot = 0.0, n_vis = 0.0;
   for (int i = i0; i < i1; i += istep) {
@@ -2449,6 +2469,9 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
       if (upd && B.vmask) upd = B.vmask[((size_t)f * NYX + c) * g.N_z + z] != 0;
       return upd;
     };
+    if (tid == 0) s_cnt = s_far = 0;
+    __syncthreads();
+    int far = 0;
     for (int p = tid; p < nv; p += NT) {
       const int v = vlist[p];
       int first = 0;
@@ -2459,7 +2482,10 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
                             vals[3] * g.delta_t);
       a_v2[p] = make_float2(vals[4] * g.delta_t, vals[5] * g.delta_t);
       a_first[p] = first;
+      if (BUF) a_view[p] = v;
+      if (vals[4] != 0.f || vals[5] != 0.f) far = 1;
     }
+    if (far) s_far = 1;
     for (int q = tid; q < 11 * ZL; q += NT) {
       const int k = q / ZL, z = q - k * ZL;
       float val = 0.f;
@@ -2480,8 +2506,8 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
     }
     if (tid < 64) magb[tid] = 0.f;
     if (tid < ZL) delta[tid] = 0.f;
-    if (tid == 0) s_cnt = 0;
     __syncthreads();
+    const bool near = s_far == 0;  // no view has bins 4 and 5: the rows are 6 bins wide
     float *xcol = xn + 4 * ZL;
     for (int ph = 0; ph < nph; ph++) {
       // the lane's slice in this phase: the one of rows lt-1..lt+1 whose index
@@ -2500,34 +2526,110 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
       const float l0 = col == 0 ? g.lap[0] : (col == 1 ? g.lap[1] : g.lap[2]);
       const float l1 = col == 0 ? g.lap[3] : (col == 1 ? g.lap[4] : g.lap[5]);
       const float l2 = col == 0 ? g.lap[6] : (col == 1 ? g.lap[7] : g.lap[8]);
-      float th1 = 0.f, th2 = 0.f;
-      int cnt = 0;
-      if (act) {
-        for (int p = grp; p < nv; p += G) {
-          const int v = vlist[p];
-          const float4 a4 = a_v4[p];
-          const float2 a2 = a_v2[p];
-          const float vals[XT_MAXA] = {a4.x, a4.y, a4.z, a4.w, a2.x, a2.y};
-          const int first = a_first[p];
-#pragma unroll
-          for (int rr = -1; rr <= XT_MAXA; rr++) {
-            const int r = first + rr;
-            if (r < 0 || r >= g.N_r) continue;
-            const float pe = xt_pc_entry(vals, rr, l0, l1, l2);
-            if (pe == 0.f) continue;
-            const size_t idx = xt_sidx(g, v, r, lt);
-            const float e1 = B.e[idx], w1 = B.w[idx];
-            const float wr = Td * __builtin_amdgcn_sqrtf(w1) * __builtin_amdgcn_rcpf(fabsf(e1));
-            const float ws = (e1 * e1 * w1 < T2) ? w1 : wr;
-            const float pw = pe * ws;
-            th2 += pe * pw;
-            th1 -= e1 * pw;
-            cnt++;
+      // the prior of the phase's slices, a neighbour to a lane, 32 lanes to a slice
+      for (int z = ph + (tid >> 5) * nph; z < g.N_z; z += (NT / 32) * nph) {
+        if (!slice_on(z)) continue;
+        const int l = tid & 31;
+        const float V = xcol[z];
+        float s1 = 0.f, s2 = 0.f;
+        bool pos = false;
+        const int k = l % 9, z2 = z + l / 9 - 1, y2 = yy + k / 3 - 1, x2 = xx + k % 3 - 1;
+        if (l < 27) {
+          if (l != 13 && z2 >= 0 && z2 < g.N_z && y2 >= 0 && y2 < g.N_y && x2 >= 0 && x2 < g.N_x) {
+            const float nb = xn[k * ZL + z2];
+            pos = nb > 0.f;
+            s2 = g.filt[l] * xt_qggmrf_ratio(V - nb, g.MRF_P, g.C_S, g.Sigma_S_Q, g.Sigma_S_Q_P);
+            s1 = s2 * nb;
           }
+        } else if (l < 29 && (l == 27 ? f > 0 : f + 1 < g.N_time)) {
+          const float nb = xn[(l - 18) * ZL + z];
+          pos = nb > 0.f;
+          s2 = g.tfilt * xt_qggmrf_ratio(V - nb, g.MRF_P, g.C_T, g.Sigma_T_Q, g.Sigma_T_Q_P);
+          s1 = s2 * nb;
+        }
+        int any = pos;
+#pragma unroll
+        for (int m = 1; m < 32; m <<= 1) {
+          s1 += __shfl_xor(s1, m);
+          s2 += __shfl_xor(s2, m);
+          any |= __shfl_xor(any, m);
+        }
+        if (l == 0) {
+          ps1[z] = s1;
+          ps2[z] = s2;
+          delta[z] = any ? 1.f : 0.f;
         }
       }
-      red1[tid] = th1;
-      red2[tid] = th2;
+      float th1 = 0.f, th2 = 0.f;
+      int cnt = 0;
+      // bins B0.. of the footprint's row, NB of them, U views in flight
+      auto theta = [&](auto b0c, auto nbc) {
+        constexpr int B0 = decltype(b0c)::value, NB = decltype(nbc)::value, U = 2;
+        for (int q0 = grp; q0 < nv; q0 += U * G) {
+          float pe[U][NB], ev[U][NB], wv[U][NB];
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            const int p = q0 + u * G;
+            float vals[XT_MAXA] = {};
+            int first = 0, v = 0;
+            if (p < nv) {
+              const float4 a4 = a_v4[p];
+              vals[0] = a4.x;
+              vals[1] = a4.y;
+              vals[2] = a4.z;
+              vals[3] = a4.w;
+              const float2 a2 = a_v2[p];
+              vals[4] = a2.x;
+              vals[5] = a2.y;
+              first = a_first[p];
+              v = BUF ? a_view[p] : vlist[p];
+            }
+            // the footprint's first bin of this row (negative where it starts off the detector)
+            const long long row = ((long long)v * g.N_r + first - 1 + B0) * g.N_t + lt;
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+              const float val = xt_pc_entry(vals, B0 + b - 1, l0, l1, l2);
+              pe[u][b] = (unsigned)(first + B0 + b - 1) < (unsigned)g.N_r ? val : 0.f;
+              // a bin outside the footprint reads nothing (or the first entry), and drops it
+              if constexpr (BUF) {
+                const uint32_t o = pe[u][b] != 0.f ? (uint32_t)((int)row + b * g.N_t) * 4u : OOB;
+                ev[u][b] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_e, o, 0, 0));
+                wv[u][b] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_w, o, 0, 0));
+              } else {
+                const size_t idx = pe[u][b] != 0.f ? (size_t)(row + b * g.N_t) : 0;
+                ev[u][b] = B.e[idx];
+                wv[u][b] = B.w[idx];
+              }
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+              const float e1 = ev[u][b], w1 = wv[u][b];
+              const float wr = Td * __builtin_amdgcn_sqrtf(w1) * __builtin_amdgcn_rcpf(fabsf(e1));
+              const float ws = (e1 * e1 * w1 < T2) ? w1 : wr;
+              const bool in = pe[u][b] != 0.f;
+              const float pw = pe[u][b] * ws;
+              th2 += in ? pe[u][b] * pw : 0.f;
+              th1 -= in ? e1 * pw : 0.f;
+              cnt += in;
+            }
+        }
+      };
+      if (act) {
+        theta(std::integral_constant<int, 0>{}, std::integral_constant<int, 6>{});
+        if (!near) theta(std::integral_constant<int, 6>{}, std::integral_constant<int, XT_MAXA - 4>{});
+      }
+#pragma unroll
+      for (int m = RL; m < 64; m <<= 1) {
+        th1 += __shfl_xor(th1, m);
+        th2 += __shfl_xor(th2, m);
+      }
+      if ((tid & 63) < RL) {
+        red1[(tid >> 6) * RL + lt] = th1;
+        red2[(tid >> 6) * RL + lt] = th2;
+      }
       if (cnt) atomicAdd(&s_cnt, cnt);
       __syncthreads();
       // the phase's slices, one thread each: theta over its three rows and the
@@ -2538,41 +2640,15 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
         for (int q = -1; q <= 1; q++) {
           const int t = z + q;
           if (t < 0 || t >= g.N_t) continue;
-          for (int gg = 0; gg < G; gg++) {
+          for (int gg = 0; gg < NT / 64; gg++) {
             T1 += red1[gg * RL + t];
             T2z += red2[gg * RL + t];
           }
         }
         const float V = xcol[z];
-        bool any_pos = false;
-        float s1 = 0.f, s2 = 0.f;
-        for (int dz = -1; dz <= 1; dz++)
-          for (int k = 0; k < 9; k++) {
-            const int l = (dz + 1) * 9 + k;
-            const int z2 = z + dz, y2 = yy + k / 3 - 1, x2 = xx + k % 3 - 1;
-            if (l == 13 || z2 < 0 || z2 >= g.N_z || y2 < 0 || y2 >= g.N_y || x2 < 0 || x2 >= g.N_x)
-              continue;
-            const float nb = xn[k * ZL + z2];
-            any_pos |= nb > 0.f;
-            const float bq =
-                g.filt[l] * xt_qggmrf_ratio(V - nb, g.MRF_P, g.C_S, g.Sigma_S_Q, g.Sigma_S_Q_P);
-            s1 += bq * nb;
-            s2 += bq;
-          }
-        if (f > 0) {
-          const float tn = xn[9 * ZL + z];
-          any_pos |= tn > 0.f;
-          const float bq = g.tfilt * xt_qggmrf_ratio(V - tn, g.MRF_P, g.C_T, g.Sigma_T_Q, g.Sigma_T_Q_P);
-          s1 += bq * tn;
-          s2 += bq;
-        }
-        if (f + 1 < g.N_time) {
-          const float tn = xn[10 * ZL + z];
-          any_pos |= tn > 0.f;
-          const float bq = g.tfilt * xt_qggmrf_ratio(V - tn, g.MRF_P, g.C_T, g.Sigma_T_Q, g.Sigma_T_Q_P);
-          s1 += bq * tn;
-          s2 += bq;
-        }
+        const bool any_pos = delta[z] != 0.f;
+        const float s1 = ps1[z], s2 = ps2[z];
+        delta[z] = 0.f;
         if (!((V == 0.f) && (iter > 1) && !any_pos)) {
           const float u = (s1 + (T2z * V) - T1) / (s2 + T2z);
           float nv2 = V + g.alpha * (u - V);
@@ -2589,18 +2665,28 @@ __global__ void __launch_bounds__(256) k_icd_lines_pc(XtGeom g, XtIcdBuffers B, 
       const float dl = act ? delta[zt] : 0.f;
       if (dl != 0.f) {
         for (int p = grp; p < nv; p += G) {
-          const int v = vlist[p];
+          const int v = BUF ? a_view[p] : vlist[p];
           const float4 a4 = a_v4[p];
           const float2 a2 = a_v2[p];
           const float vals[XT_MAXA] = {a4.x, a4.y, a4.z, a4.w, a2.x, a2.y};
           const int first = a_first[p];
+          const long long row = ((long long)v * g.N_r + first - 1) * g.N_t + lt;
+          auto apply = [&](auto b0c, auto nbc) {
+            constexpr int B0 = decltype(b0c)::value;
 #pragma unroll
-          for (int rr = -1; rr <= XT_MAXA; rr++) {
-            const int r = first + rr;
-            if (r < 0 || r >= g.N_r) continue;
-            const float pe = xt_pc_entry(vals, rr, l0, l1, l2);
-            if (pe != 0.f) atomicAdd(&B.e[xt_sidx(g, v, r, lt)], -(pe * dl));
-          }
+            for (int b = B0; b < B0 + decltype(nbc)::value; b++) {
+              const float val = xt_pc_entry(vals, b - 1, l0, l1, l2);
+              const float pe = (unsigned)(first + b - 1) < (unsigned)g.N_r ? val : 0.f;
+              if constexpr (BUF)
+                (void)__builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(
+                    -(pe * dl), rs_e, pe != 0.f ? (uint32_t)((int)row + b * g.N_t) * 4u : OOB, 0, 0);
+              else if (pe != 0.f)
+                atomicAdd(&B.e[row + b * g.N_t], -(pe * dl));
+            }
+          };
+          apply(std::integral_constant<int, 0>{}, std::integral_constant<int, 6>{});
+          if (!near)
+            apply(std::integral_constant<int, 6>{}, std::integral_constant<int, XT_MAXA - 4>{});
         }
       }
       // the next phase's theta reads these e entries

@@ -736,6 +736,18 @@ static int launch_pass(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
   return XT_OK;
 }
 
+// dynamic LDS of k_icd_lines_pc with nt threads: with 256, never more than icd_lds_bytes()
+static size_t pc_lds_bytes(const XtGeom &g, int ZL, int nt) {
+  return (size_t)g.max_views * (sizeof(float4) + sizeof(float2) + (nt > 256 ? 2 : 1) * sizeof(int)) +
+         ((size_t)nt / 32 * ZL + 14 * ZL + 64) * sizeof(float);
+}
+
+template <int ZL, int NT>
+static void pc_go(xt_icd_state *s, const XtIcdBuffers &B, const XtIcdLaunch &L, int gx) {
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_icd_lines_pc<ZL, NT>), dim3(gx, s->g.N_time), dim3(NT),
+                     pc_lds_bytes(s->g, ZL, NT), s->st, s->g, B, L);
+}
+
 static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
   XtIcdBuffers B = buffers_of(s);
   size_t lds = icd_lds_bytes(s->g, s->ZL, B.at_vals != nullptr, s->nt);
@@ -761,12 +773,17 @@ static int launch_icd(xt_icd_state *s, const XtIcdLaunch &L, int gx) {
     return XT_OK;
   }
   if (s->g.pc) {
-    const dim3 grid(gx, s->g.N_time), block(256);
+    // 16 waves a line up to a line per CU (the chip's 256), else 4; 4 too where the wider
+    // group's partial sums do not fit beside the footprints, and for a sinogram that the
+    // 32-bit offsets of its buffer loads do not reach
+    const bool wide = (long long)gx * s->g.N_time <= 256 &&
+                      (size_t)s->g.N_p * s->g.N_r * s->g.N_t * sizeof(float) <= (size_t)1 << 31 &&
+                      pc_lds_bytes(s->g, s->ZL, 1024) <= 64 * 1024;
     switch (s->ZL) {
-      case 8: hipLaunchKernelGGL(k_icd_lines_pc<8>, grid, block, lds, s->st, s->g, B, L); break;
-      case 16: hipLaunchKernelGGL(k_icd_lines_pc<16>, grid, block, lds, s->st, s->g, B, L); break;
-      case 32: hipLaunchKernelGGL(k_icd_lines_pc<32>, grid, block, lds, s->st, s->g, B, L); break;
-      default: hipLaunchKernelGGL(k_icd_lines_pc<64>, grid, block, lds, s->st, s->g, B, L); break;
+      case 8: wide ? pc_go<8, 1024>(s, B, L, gx) : pc_go<8, 256>(s, B, L, gx); break;
+      case 16: wide ? pc_go<16, 1024>(s, B, L, gx) : pc_go<16, 256>(s, B, L, gx); break;
+      case 32: wide ? pc_go<32, 1024>(s, B, L, gx) : pc_go<32, 256>(s, B, L, gx); break;
+      default: wide ? pc_go<64, 1024>(s, B, L, gx) : pc_go<64, 256>(s, B, L, gx); break;
     }
     XT_HIP(hipGetLastError());
     if (s->timing) XT_HIP(hipEventRecord(e1, s->st));
