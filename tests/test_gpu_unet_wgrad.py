@@ -33,3 +33,21 @@ def test_gradients_at_tile_edges(shape):
     errs = {name: rel(g[sl], wg[sl]) for name, sl in uo.layer_slices()}
     print(f"  worst gradient block: {max(errs.items(), key=lambda e: e[1])}")
     assert max(errs.values()) <= 3e-2, errs
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 32), (24, 24, 16), (80, 16, 64)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_forward_at_tile_edges(shape):
+    """32, 16 and 64 voxels along d2: every width of the marching convolution's tile, rows
+    past the volume, several segments of d0 (the gradients' shapes have 8 along d2).
+    Relative L2 error of the network's own part <= 1e-2, as at 16 x 16 x 8."""
+    print(f"[gpu] unet forward {shape}", flush=True)
+    p = _params(8)
+    x, _ = _volume(9, shape)
+    with xt_hip.UNet(shape, SCALE, seed=0) as net:
+        net.set_params(p)
+        got = net.forward(x)
+    want = uo.UNet(p, SCALE, bf16=True).forward(x)
+    e = rel((got.astype(np.float64) - x) * SCALE, (want - x) * SCALE)
+    print(f"  rel L2 of the residual: {e:.2e}")
+    assert e <= 1e-2

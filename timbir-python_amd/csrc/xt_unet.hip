@@ -160,21 +160,20 @@ __global__ void __launch_bounds__(256) k_conv3(const bf16_t *__restrict__ in, in
   }
 }
 
-// LDS-tiled variant for Ci % 16 == 0: a workgroup's 64*MB voxels form a TY x TX
-// tile of one d0-plane (TX along d2); per chunk of CC input channels the tile
+// LDS-tiled variant for Ci % 32 == 0: a workgroup's 64*MB voxels form a TY x TX
+// tile of one d0-plane (TX along d2); per chunk of 32 input channels the tile
 // and its one-voxel halo in d0, d1 and d2 are staged in LDS once and every
 // tap's A fragment is read from there (the direct kernel reads each input 27
-// times from L2).  K order: channel chunks outer, taps inner (CC = 32: one tap
-// per MFMA K-step; CC = 16: two).  TY | d1 and TX | d2.
-template <int MB, int NB, int CC>
+// times from L2).  K order: channel chunks outer, taps inner, one tap per MFMA
+// K-step.  TY | d1 and TX | d2.
+template <int MB, int NB>
 __global__ void __launch_bounds__(256) k_conv3_lds(const bf16_t *__restrict__ in, int Ci,
                                                    const bf16_t *__restrict__ W, int Kpad,
                                                    const float *__restrict__ bias, int Co, int d0,
                                                    int d1, int d2, int TY, int TX,
                                                    bf16_t *__restrict__ out, int relu,
                                                    const bf16_t *__restrict__ mask) {
-  constexpr int CP = CC + 8;  // padded channel stride of a staged voxel (bf16)
-  constexpr int TPS = 32 / CC;
+  constexpr int CC = 32, CP = CC + 8;  // channels of a chunk, padded stride of a staged voxel
   extern __shared__ uint4 lds4[];
   bf16_t *tile = (bf16_t *)lds4;  // [3][TY+2][TX+2][CP]
   const int P = d1 * d2;
@@ -216,21 +215,19 @@ __global__ void __launch_bounds__(256) k_conv3_lds(const bf16_t *__restrict__ in
       *(uint4 *)(tile + (size_t)hv * CP + 8 * c8) = v;
     }
     __syncthreads();
-    for (int t0 = 0; t0 < 27; t0 += TPS) {
-      const int tap = t0 + (TPS == 2 ? (g >> 1) : 0);
-      const int cg = (TPS == 2 ? (g & 1) : g) * 8;
-      const bool tok = tap < 27;
+    for (int tap = 0; tap < 27; tap++) {
+      const int cg = g * 8;
       const int a0 = tap / 9, a1 = (tap / 3) % 3, a2 = tap % 3;  // halo offsets 0..2
       bf16x8 a[MB], b[NB];
 #pragma unroll
       for (int mb = 0; mb < MB; mb++) {
         const int hv = (a0 * HY + ty[mb] + a1) * HX + tx[mb] + a2;
-        a[mb] = as_bf16x8((tok && rok[mb]) ? *(const uint4 *)(tile + (size_t)hv * CP + cg) : zero4);
+        a[mb] = as_bf16x8(rok[mb] ? *(const uint4 *)(tile + (size_t)hv * CP + cg) : zero4);
       }
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
         const int co = n0 + nb * 16 + r;
-        b[nb] = as_bf16x8((tok && co < Co)
+        b[nb] = as_bf16x8(co < Co
                               ? *(const uint4 *)(W + (size_t)co * Kpad + (size_t)tap * Ci + c0 + cg)
                               : zero4);
       }
@@ -259,6 +256,123 @@ __global__ void __launch_bounds__(256) k_conv3_lds(const bf16_t *__restrict__ in
         if (mask && !bf_pos(mask[v * Co + co])) val = 0.f;
         out[v * Co + co] = f2bf(val);
       }
+  }
+}
+
+// 3x3x3 conv of Ci = 16 * NC channels (NC 1 or 3: the layers at full resolution, forward
+// and backward-data): a workgroup keeps 16 * NC x 16 weights in registers and marches along
+// d0 over a tile of TY x TX voxels (256 of them, TX = 1 << ltx along d2).  The input planes
+// p-1, p, p+1 with their halo lie in a ring of four in LDS, so each is read once per tile
+// (4/3 of the voxels, not 27 times or 3 * 4/3) while the one after next is under way to
+// registers; halves of 8 channels are laid out apart, so that a fragment's 16 voxels are
+// 256 consecutive bytes.  K order: chunks of 16 channels, in each the taps by pairs, as
+// k_conv3 with Ci = 16 (bit for bit the same sums).  The product is taken as weights x
+// voxels: a lane ends with 4 channels of one voxel and stores them together.  Bound by
+// the LDS reads of fragments (one per MFMA, 8 cycles of a CU each).  512 x 512 x 32:
+//   48->16   755 us; 1580 with a tile of one plane staged per channel chunk (3 * 4/3 reads)
+//   16->16   175 us; 521 with fragments read from L2 for every tap
+constexpr int MARCH_HV = 344;  // staged voxels of a plane, at most 340, up to a half's stride
+
+template <int NC>
+__global__ void __launch_bounds__(512, 2) k_conv3_march(
+    const bf16_t *__restrict__ in, const bf16_t *__restrict__ W, int Kpad,
+    const float *__restrict__ bias, int Co, int d0, int d1, int d2, int ltx, int seg,
+    bf16_t *__restrict__ out, int relu, const bf16_t *__restrict__ mask) {
+  constexpr int Ci = 16 * NC, C8 = 2 * NC, PL = C8 * MARCH_HV, NP = (340 * C8 + 511) / 512;
+  extern __shared__ uint4 ring[];  // [4][C8][MARCH_HV]
+  const int TX = 1 << ltx, TY = 256 >> ltx, HX = TX + 2, HV = (TY + 2) * HX, P = d1 * d2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const bool odd = g >> 1;  // the second tap of a pair
+  const int ntx = d2 >> ltx;
+  const int x0 = (blockIdx.x % ntx) << ltx, y0 = blockIdx.x / ntx * TY;
+  const int n0 = blockIdx.y * 16;
+  const int pb = blockIdx.z * seg, pe = min(pb + seg, d0);
+  const uint4 zero4 = {0u, 0u, 0u, 0u};
+  // this thread's pieces (8 channels of a voxel) of a plane
+  int pix[NP], dst[NP];
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const int q = tid + i * 512, hv = q / C8, c8 = q - hv * C8;
+    const int yy = y0 + hv / HX - 1, xx = x0 + hv % HX - 1;
+    const bool ok = hv < HV && (unsigned)yy < (unsigned)d1 && (unsigned)xx < (unsigned)d2;
+    pix[i] = ok ? yy * d2 + xx : -1;
+    dst[i] = hv < HV ? c8 * MARCH_HV + hv : -1;
+  }
+  uint4 v[NP];
+  auto load = [&](int p) {
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      v[i] = zero4;
+      if ((unsigned)p < (unsigned)d0 && pix[i] >= 0)
+        v[i] = *(const uint4 *)(in + (size_t)(p * P + pix[i]) * Ci + (tid + i * 512) % C8 * 8);
+    }
+  };
+  auto store = [&](int p) {
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+      if (dst[i] >= 0) ring[((p + 4) & 3) * PL + dst[i]] = v[i];
+  };
+  for (int p = pb - 1; p <= pb + 1; p++) {
+    load(p);
+    store(p);
+  }
+  uint4 w[NC][14];
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int s = 0; s < 14; s++) {
+      const int tap = 2 * s + odd;
+      w[c][s] = tap < 27 ? *(const uint4 *)(W + (size_t)(n0 + r) * Kpad + tap * Ci + c * 16 + (g & 1) * 8)
+                         : zero4;
+    }
+  // the wave's two blocks of 16 voxels, hv of their taps' first corner
+  const int m0 = wave * 32 + r, m1 = m0 + 16;
+  const int hv0 = (m0 >> ltx) * HX + (m0 & (TX - 1)), hv1 = (m1 >> ltx) * HX + (m1 & (TX - 1));
+  const int base = (g & 1) * MARCH_HV + hv0, step = hv1 - hv0;
+  float bv[4] = {0.f, 0.f, 0.f, 0.f};
+  if (bias)
+#pragma unroll
+    for (int i = 0; i < 4; i++) bv[i] = bias[n0 + g * 4 + i];
+  for (int p = pb; p < pe; p++) {
+    __syncthreads();  // planes p-1..p+1 are staged; nobody reads plane p-2 any more
+    if (p + 1 < pe) load(p + 2);
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int s = 0; s < 14; s++) {
+        // both taps' offsets are the same for all lanes; tap 27 does not exist
+        const int t0 = 2 * s, t1 = s == 13 ? 26 : 2 * s + 1;
+        const int o0 = ((p + 3 + t0 / 9) & 3) * PL + t0 / 3 % 3 * HX + t0 % 3;
+        const int o1 = ((p + 3 + t1 / 9) & 3) * PL + t1 / 3 % 3 * HX + t1 % 3;
+        const int q = base + (odd ? o1 : o0) + c * 2 * MARCH_HV;
+        uint4 b0 = ring[q], b1 = ring[q + step];
+        if (s == 13 && odd) b0 = b1 = zero4;
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[c][s]), as_bf16x8(b0), acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[c][s]), as_bf16x8(b1), acc[1], 0, 0, 0);
+      }
+    if (p + 1 < pe) store(p + 2);
+    // lane holds voxel r and channels g*4+i of each block
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++) {
+      const int m = mb ? m1 : m0, yy = y0 + (m >> ltx), xx = x0 + (m & (TX - 1));
+      if (yy >= d1) continue;
+      const size_t o = (size_t)(p * P + yy * d2 + xx) * Co + n0 + g * 4;
+      uint2 mk = {0u, 0u};
+      if (mask) mk = *(const uint2 *)(mask + o);
+      bf16_t e[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float val = acc[mb][i] + bv[i];
+        if (relu) val = fmaxf(val, 0.f);
+        const bf16_t k = (bf16_t)((i < 2 ? mk.x : mk.y) >> (16 * (i & 1)));
+        if (mask && !bf_pos(k)) val = 0.f;
+        e[i] = f2bf(val);
+      }
+      *(uint2 *)(out + o) =
+          make_uint2(e[0] | ((uint32_t)e[1] << 16), e[2] | ((uint32_t)e[3] << 16));
+    }
   }
 }
 
@@ -760,7 +874,6 @@ struct xt_unet {
   float *stage = nullptr;  // [2][V0] host-call staging (input, target/output)
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   double fwd_ms = 0, bwd_ms = 0;
-  bool lds_conv = true;  // LDS-tiled convolutions where Ci % 16 == 0 and Ci >= 32
 };
 
 namespace {
@@ -784,47 +897,53 @@ int pow2_divisor(int n, int cap) {  // largest power of two dividing n, at most 
   return p;
 }
 
+// dynamic LDS of k_conv3_march: four planes
+size_t march_lds(int Ci) { return (size_t)4 * (Ci / 8) * MARCH_HV * sizeof(uint4); }
+
 void launch_conv(xt_unet *u, hipStream_t st, const bf16_t *in, int Ci, const bf16_t *W, int Kpad,
                  const float *bias, int Co, const int *d, bf16_t *out, int relu,
                  const bf16_t *mask) {
   const int V = d[0] * d[1] * d[2];
   const int NB = (Co % 64 == 0) ? 4 : (Co % 32 == 0) ? 2 : 1;
-  // LDS tiles pay from 32 input channels on: with 16 the 4x halo staging costs
-  // more than the L2 re-reads it saves (16->16 at 512x512x32: 785 against 547 us)
-  if (Ci % 16 == 0 && Ci >= 32 && u->lds_conv) {
-    const int CC = (Ci % 32 == 0) ? 32 : 16;
-    const int MBl = (NB == 1 && CC == 16) ? 4 : 2;
-    const int TX = pow2_divisor(d[2], std::min(32, 64 * MBl));
-    const int TY = pow2_divisor(d[1], 64 * MBl / TX);
-    const size_t lds = (size_t)3 * (TY + 2) * (TX + 2) * (CC + 8) * sizeof(bf16_t);
+  if ((Ci == 16 || Ci == 48) && Co % 16 == 0 && d[2] % 8 == 0) {
+    // a workgroup (16 channels) or two thirds of one (48) a CU over two rounds, but 8
+    // planes at least: a segment stages two more than it computes
+    const int TX = pow2_divisor(d[2], 32), ltx = __builtin_ctz(TX), TY = 256 / TX;
+    const int nt = (d[2] / TX) * ((d[1] + TY - 1) / TY) * (Co / 16);
+    const int nseg = std::max(1, std::min((Ci == 16 ? 1536 : 512) / nt, d[0] / 8));
+    const int seg = (d[0] + nseg - 1) / nseg;
+    const dim3 grid((d[2] / TX) * ((d[1] + TY - 1) / TY), Co / 16, (d[0] + seg - 1) / seg);
+    const size_t lds = march_lds(Ci);
+    if (Ci == 16)
+      hipLaunchKernelGGL((k_conv3_march<1>), grid, dim3(512), lds, st, in, W, Kpad, bias, Co, d[0],
+                         d[1], d[2], ltx, seg, out, relu, mask);
+    else
+      hipLaunchKernelGGL((k_conv3_march<3>), grid, dim3(512), lds, st, in, W, Kpad, bias, Co, d[0],
+                         d[1], d[2], ltx, seg, out, relu, mask);
+    return;
+  }
+  if (Ci % 32 == 0) {
+    const int TX = pow2_divisor(d[2], 32), TY = pow2_divisor(d[1], 128 / TX);
+    const size_t lds = (size_t)3 * (TY + 2) * (TX + 2) * (32 + 8) * sizeof(bf16_t);
     dim3 grid(d[0] * (d[1] / TY) * (d[2] / TX), Co / (16 * NB));
-#define UN_LDS(MB_, NB_, CC_)                                                                     \
-  hipLaunchKernelGGL((k_conv3_lds<MB_, NB_, CC_>), grid, dim3(256), lds, st, in, Ci, W, Kpad, bias, \
-                     Co, d[0], d[1], d[2], TY, TX, out, relu, mask)
-    if (NB == 1 && CC == 16) UN_LDS(4, 1, 16);
-    else if (NB == 1) UN_LDS(2, 1, 32);
-    else if (NB == 2 && CC == 16) UN_LDS(2, 2, 16);
-    else if (NB == 2) UN_LDS(2, 2, 32);
-    else if (CC == 16) UN_LDS(2, 4, 16);
-    else UN_LDS(2, 4, 32);
+#define UN_LDS(NB_)                                                                                \
+  hipLaunchKernelGGL((k_conv3_lds<2, NB_>), grid, dim3(256), lds, st, in, Ci, W, Kpad, bias, Co,   \
+                     d[0], d[1], d[2], TY, TX, out, relu, mask)
+    if (NB == 1) UN_LDS(1);
+    else if (NB == 2) UN_LDS(2);
+    else UN_LDS(4);
 #undef UN_LDS
     return;
   }
+  // the stem; and 16 -> 32 channels at half resolution where d2 has no factor 8
   const int MB = 8 / NB;
   dim3 grid((V + 64 * MB - 1) / (64 * MB), Co / (16 * NB));
-  if (Ci % 8 != 0) {
+  if (NB == 1)
     hipLaunchKernelGGL((k_conv3<false, 8, 1>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
                        d[0], d[1], d[2], out, relu, mask);
-  } else if (NB == 1) {
-    hipLaunchKernelGGL((k_conv3<true, 8, 1>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
-                       d[0], d[1], d[2], out, relu, mask);
-  } else if (NB == 2) {
+  else
     hipLaunchKernelGGL((k_conv3<true, 4, 2>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
                        d[0], d[1], d[2], out, relu, mask);
-  } else {
-    hipLaunchKernelGGL((k_conv3<true, 2, 4>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
-                       d[0], d[1], d[2], out, relu, mask);
-  }
 }
 
 void launch_wgrad(hipStream_t st, const bf16_t *in, int Ci, const bf16_t *gout, int Co,
@@ -1043,6 +1162,14 @@ extern "C" int xt_unet_create(int32_t d0, int32_t d1, int32_t d2, float scale, u
       return fail(xt_report_error(XT_E_HIP, "U-Net allocation of %zu bytes: %s",           \
                                   (size_t)(bytes), hipGetErrorString(_e)));                \
   } while (0)
+  {
+    const hipError_t e = hipFuncSetAttribute((const void *)k_conv3_march<3>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)march_lds(48));
+    if (e != hipSuccess)
+      return fail(xt_report_error(XT_E_HIP, "U-Net: %zu bytes of LDS: %s", march_lds(48),
+                                  hipGetErrorString(e)));
+  }
   UN_ALLOC(u->params, off * sizeof(float));
   UN_ALLOC(u->wbuf, wcount * sizeof(bf16_t) + 256);
   {
