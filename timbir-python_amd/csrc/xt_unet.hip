@@ -56,10 +56,9 @@ __device__ inline bf16x8 as_bf16x8(uint4 q) { return __builtin_bit_cast(bf16x8, 
 // ---------------------------------------------------------------------------
 // 3x3x3 conv, forward (also backward-data).  Workgroup = 4 waves; a wave
 // computes 16*MB voxels x 16*NB output channels.  K runs over kk = tap*Ci + ci
-// padded to Kpad (multiple of 32) with zero weights.  VEC: Ci % 8 == 0 (one
-// 16-byte load per lane and fragment), else element gathers (the 1-channel
-// stem).  Optional epilogue: + bias, ReLU, x (mask > 0).
-template <bool VEC, int MB, int NB>
+// padded to Kpad (multiple of 32) with zero weights; Ci % 8 == 0 (one 16-byte load
+// per lane and fragment).  Optional epilogue: + bias, ReLU, x (mask > 0).
+template <int MB, int NB>
 __global__ void __launch_bounds__(256) k_conv3(const bf16_t *__restrict__ in, int Ci,
                                                const bf16_t *__restrict__ W, int Kpad,
                                                const float *__restrict__ bias, int Co, int d0,
@@ -84,50 +83,25 @@ __global__ void __launch_bounds__(256) k_conv3(const bf16_t *__restrict__ in, in
   for (int mb = 0; mb < MB; mb++)
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int Ktot = 27 * Ci;
   const uint4 zero4 = {0u, 0u, 0u, 0u};
   int tap = (g * 8) / Ci, ci = g * 8 - tap * Ci;  // (tap, ci) of kk = k0 + g*8
   for (int k0 = 0; k0 < Kpad; k0 += 32) {
     bf16x8 a[MB], b[NB];
-    if constexpr (VEC) {
-      const int a0 = tap / 9 - 1, a1 = (tap / 3) % 3 - 1, a2 = tap % 3 - 1;
-      const bool tok = tap < 27;
-      const int off = a0 * P + a1 * d2 + a2;
+    const int a0 = tap / 9 - 1, a1 = (tap / 3) % 3 - 1, a2 = tap % 3 - 1;
+    const bool tok = tap < 27;
+    const int off = a0 * P + a1 * d2 + a2;
 #pragma unroll
-      for (int mb = 0; mb < MB; mb++) {
-        const int p0 = c0[mb] + a0, p1 = c1[mb] + a1, p2 = c2[mb] + a2;
-        const bool ok = tok && (unsigned)p0 < (unsigned)d0 && (unsigned)p1 < (unsigned)d1 &&
-                        (unsigned)p2 < (unsigned)d2;
-        const int v = m0 + mb * 16 + r;
-        a[mb] = as_bf16x8(ok ? *(const uint4 *)(in + (size_t)(v + off) * Ci + ci) : zero4);
-      }
-      ci += 32;
-      while (ci >= Ci) {
-        ci -= Ci;
-        tap++;
-      }
-    } else {
-      const int kk = k0 + g * 8;
-#pragma unroll
-      for (int mb = 0; mb < MB; mb++) {
-        const int v = m0 + mb * 16 + r;
-        uint16_t e[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const int kj = kk + j, t = kj / Ci, cj = kj - t * Ci;
-          const int a0 = t / 9 - 1, a1 = (t / 3) % 3 - 1, a2 = t % 3 - 1;
-          const int p0 = c0[mb] + a0, p1 = c1[mb] + a1, p2 = c2[mb] + a2;
-          const bool ok = kj < Ktot && (unsigned)p0 < (unsigned)d0 && (unsigned)p1 < (unsigned)d1 &&
-                          (unsigned)p2 < (unsigned)d2;
-          e[j] = ok ? in[(size_t)(v + a0 * P + a1 * d2 + a2) * Ci + cj] : (uint16_t)0;
-        }
-        uint4 q;
-        q.x = e[0] | ((uint32_t)e[1] << 16);
-        q.y = e[2] | ((uint32_t)e[3] << 16);
-        q.z = e[4] | ((uint32_t)e[5] << 16);
-        q.w = e[6] | ((uint32_t)e[7] << 16);
-        a[mb] = as_bf16x8(q);
-      }
+    for (int mb = 0; mb < MB; mb++) {
+      const int p0 = c0[mb] + a0, p1 = c1[mb] + a1, p2 = c2[mb] + a2;
+      const bool ok = tok && (unsigned)p0 < (unsigned)d0 && (unsigned)p1 < (unsigned)d1 &&
+                      (unsigned)p2 < (unsigned)d2;
+      const int v = m0 + mb * 16 + r;
+      a[mb] = as_bf16x8(ok ? *(const uint4 *)(in + (size_t)(v + off) * Ci + ci) : zero4);
+    }
+    ci += 32;
+    while (ci >= Ci) {
+      ci -= Ci;
+      tap++;
     }
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
@@ -270,7 +244,7 @@ __global__ void __launch_bounds__(256) k_conv3_lds(const bf16_t *__restrict__ in
 // voxels: a lane ends with 4 channels of one voxel and stores them together.  Bound by
 // the LDS reads of fragments (one per MFMA, 8 cycles of a CU each).  512 x 512 x 32:
 //   48->16   755 us; 1580 with a tile of one plane staged per channel chunk (3 * 4/3 reads)
-//   16->16   175 us; 521 with fragments read from L2 for every tap
+//   16->16   180 us; 521 with fragments read from L2 for every tap
 constexpr int MARCH_HV = 344;  // staged voxels of a plane, at most 340, up to a half's stride
 
 template <int NC>
@@ -376,109 +350,65 @@ __global__ void __launch_bounds__(512, 2) k_conv3_march(
   }
 }
 
-// Weight gradient of the one-channel stem: M = output channels (16*MBo per wave), N = kk
-// columns (16*NBk per wave), K = voxels in steps of 32.  Each workgroup reduces one chunk of
-// voxels (split over its 4 waves) and adds its partial tile to dW with FP32
-// atomics.
-template <int MBo, int NBk>
-__global__ void __launch_bounds__(256) k_conv3_wgrad(const bf16_t *__restrict__ in, int Ci,
-                                                     const bf16_t *__restrict__ gout, int Co, int d0,
-                                                     int d1, int d2, int vchunk,
-                                                     float *__restrict__ dW) {
-  const int V = d0 * d1 * d2, P = d1 * d2;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Forward of the one-channel stem (27 taps: one MFMA K-step, in k_conv3's order of taps):
+// a workgroup stages STEM_SEG + 2 planes of a TY x TX tile (as k_conv3_march) with their
+// halo at once and each lane gathers its 8 taps from there.  Gathered from memory with a
+// bounds check per tap it took 456 us at 512 x 512 x 32.
+constexpr int STEM_SEG = 32;
+
+__global__ void __launch_bounds__(512) k_stem(const bf16_t *__restrict__ in,
+                                              const bf16_t *__restrict__ W, int Kpad,
+                                              const float *__restrict__ bias, int Co, int d0, int d1,
+                                              int d2, int ltx, bf16_t *__restrict__ out) {
+  __shared__ bf16_t pl[(STEM_SEG + 2) * MARCH_HV];
+  const int TX = 1 << ltx, TY = 256 >> ltx, HX = TX + 2, HV = (TY + 2) * HX, P = d1 * d2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int co0 = blockIdx.y * (16 * MBo), kk0 = blockIdx.z * (16 * NBk);
-  const int Ktot = 27 * Ci;
-  const int wchunk = vchunk / 4;
-  const int vbeg = blockIdx.x * vchunk + wave * wchunk;
-  const int vend = min(vbeg + wchunk, V);
-  if (vbeg >= vend) return;
-  int ka0[NBk], ka1[NBk], ka2[NBk], kci[NBk];
-  bool kok[NBk];
-#pragma unroll
-  for (int nb = 0; nb < NBk; nb++) {
-    const int kk = kk0 + nb * 16 + r;
-    kok[nb] = kk < Ktot;
-    const int t = kok[nb] ? kk / Ci : 13;
-    kci[nb] = kok[nb] ? kk - t * Ci : 0;
-    ka0[nb] = t / 9 - 1;
-    ka1[nb] = (t / 3) % 3 - 1;
-    ka2[nb] = t % 3 - 1;
-  }
-  f32x4 acc[MBo][NBk];
-#pragma unroll
-  for (int mb = 0; mb < MBo; mb++)
-#pragma unroll
-    for (int nb = 0; nb < NBk; nb++) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int v0 = vbeg; v0 < vend; v0 += 32) {
-    // this lane's 8 voxels: v0 + g*8 + j
-    int v = v0 + g * 8;
-    int p0 = v / P, p1 = (v / d2) % d1, p2 = v % d2;
-    uint16_t ea[MBo][8], eb[NBk][8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const bool vok = v < vend;
-#pragma unroll
-      for (int mb = 0; mb < MBo; mb++) {
-        const int co = co0 + mb * 16 + r;
-        ea[mb][j] = (vok && co < Co) ? gout[(size_t)v * Co + co] : (uint16_t)0;
-      }
-#pragma unroll
-      for (int nb = 0; nb < NBk; nb++) {
-        const int q0 = p0 + ka0[nb], q1 = p1 + ka1[nb], q2 = p2 + ka2[nb];
-        const bool ok = vok && kok[nb] && (unsigned)q0 < (unsigned)d0 &&
-                        (unsigned)q1 < (unsigned)d1 && (unsigned)q2 < (unsigned)d2;
-        eb[nb][j] = ok ? in[(size_t)(v + ka0[nb] * P + ka1[nb] * d2 + ka2[nb]) * Ci + kci[nb]]
-                       : (uint16_t)0;
-      }
-      v++;
-      if (++p2 == d2) {
-        p2 = 0;
-        if (++p1 == d1) {
-          p1 = 0;
-          p0++;
-        }
-      }
+  const int ntx = d2 >> ltx;
+  const int x0 = (blockIdx.x % ntx) << ltx, y0 = blockIdx.x / ntx * TY;
+  const int n0 = blockIdx.y * 16, pb = blockIdx.z * STEM_SEG, np = min(STEM_SEG, d0 - pb);
+  if (tid < HV) {
+    const int yy = y0 + tid / HX - 1, xx = x0 + tid % HX - 1;
+    const bool ok = (unsigned)yy < (unsigned)d1 && (unsigned)xx < (unsigned)d2;
+    for (int k = 0; k < np + 2; k++) {
+      const int p = pb + k - 1;
+      bf16_t e = 0;
+      if (ok && (unsigned)p < (unsigned)d0) e = in[(size_t)p * P + yy * d2 + xx];
+      pl[k * MARCH_HV + tid] = e;
     }
-    bf16x8 a[MBo], b[NBk];
-#pragma unroll
-    for (int mb = 0; mb < MBo; mb++) {
-      uint4 q;
-      q.x = ea[mb][0] | ((uint32_t)ea[mb][1] << 16);
-      q.y = ea[mb][2] | ((uint32_t)ea[mb][3] << 16);
-      q.z = ea[mb][4] | ((uint32_t)ea[mb][5] << 16);
-      q.w = ea[mb][6] | ((uint32_t)ea[mb][7] << 16);
-      a[mb] = as_bf16x8(q);
-    }
-#pragma unroll
-    for (int nb = 0; nb < NBk; nb++) {
-      uint4 q;
-      q.x = eb[nb][0] | ((uint32_t)eb[nb][1] << 16);
-      q.y = eb[nb][2] | ((uint32_t)eb[nb][3] << 16);
-      q.z = eb[nb][4] | ((uint32_t)eb[nb][5] << 16);
-      q.w = eb[nb][6] | ((uint32_t)eb[nb][7] << 16);
-      b[nb] = as_bf16x8(q);
-    }
-#pragma unroll
-    for (int mb = 0; mb < MBo; mb++)
-#pragma unroll
-      for (int nb = 0; nb < NBk; nb++)
-        acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mb], b[nb], acc[mb][nb], 0, 0, 0);
   }
-  // lane holds column kk0+nb*16+r and rows co0+mb*16+g*4+i
+  const bf16x8 w = as_bf16x8(*(const uint4 *)(W + (size_t)(n0 + r) * Kpad + g * 8));
+  const int m0 = wave * 32 + r, m1 = m0 + 16;
+  const int hv0 = (m0 >> ltx) * HX + (m0 & (TX - 1)), hv1 = (m1 >> ltx) * HX + (m1 & (TX - 1));
+  int off[8];  // the lane's taps; those past the last (g = 3) are cleared below
 #pragma unroll
-  for (int nb = 0; nb < NBk; nb++) {
-    if (!kok[nb]) continue;
-    const int kk = kk0 + nb * 16 + r;
-#pragma unroll
-    for (int mb = 0; mb < MBo; mb++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int co = co0 + mb * 16 + g * 4 + i;
-        if (co < Co) atomicAdd(dW + (size_t)co * Ktot + kk, acc[mb][nb][i]);
-      }
+  for (int j = 0; j < 8; j++) {
+    const int t = min(g * 8 + j, 26);
+    off[j] = t / 9 * MARCH_HV + t / 3 % 3 * HX + t % 3;
   }
+  float bv[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) bv[i] = bias[n0 + g * 4 + i];
+  __syncthreads();
+  for (int k = 0; k < np; k++)
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++) {
+      const int m = mb ? m1 : m0, yy = y0 + (m >> ltx), xx = x0 + (m & (TX - 1));
+      const bf16_t *src = pl + k * MARCH_HV + (mb ? hv1 : hv0);
+      uint32_t e[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) e[j] = src[off[j]];
+      uint4 q = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
+      if (g == 3) q = make_uint4(q.x, q.y & 0xffffu, 0u, 0u);
+      const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, as_bf16x8(q),
+                                                                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      if (yy >= d1) continue;
+      bf16_t o[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) o[i] = f2bf(fmaxf(acc[i] + bv[i], 0.f));
+      *(uint2 *)(out + (size_t)((pb + k) * P + yy * d2 + xx) * Co + n0 + g * 4) =
+          make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+    }
 }
 
 // Weight gradient of a layer with Ci and Co multiples of 16: a workgroup takes 16 input
@@ -499,9 +429,32 @@ constexpr int WG_ROWS = 64;
 __device__ inline uint32_t wg_lo(uint32_t a, uint32_t b) { return (a & 0xffffu) | (b << 16); }
 __device__ inline uint32_t wg_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 
+// the 8 bf16 of q, by pairs
+__device__ inline float wg_sum(uint4 q) {
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t w = k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w;
+    s += __uint_as_float(w << 16) + __uint_as_float(w & 0xffff0000u);
+  }
+  return s;
+}
+
+// db[r] += the sums of the 16 lanes' channels over the workgroup; red: 64 floats
+__device__ inline void wg_bias(float s, float *red, float *db) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  s += __shfl_xor(s, 16);
+  s += __shfl_xor(s, 32);
+  __syncthreads();  // red has been read
+  if (lane < 16) red[wave * 16 + lane] = s;
+  __syncthreads();
+  if (threadIdx.x < 16)
+    atomicAdd(db + lane, (red[lane] + red[16 + lane]) + (red[32 + lane] + red[48 + lane]));
+}
+
 __global__ void __launch_bounds__(256, 3) k_conv3_wgrad_tile(
     const bf16_t *__restrict__ in, int Ci, const bf16_t *__restrict__ gout, int Co, int d0, int d1,
-    int d2, int lt2, int n1, int n2, int ntiles, float *__restrict__ dW) {
+    int d2, int lt2, int n1, int n2, int ntiles, float *__restrict__ dW, float *__restrict__ db) {
   extern __shared__ uint4 wg_smem[];
   const int T2 = 1 << lt2, T0 = WG_ROWS >> lt2, W2 = T2 + 2, NR = (T0 + 2) * W2;
   uint4 *gm = wg_smem;                       // [WG_ROWS][16] gradients
@@ -513,6 +466,7 @@ __global__ void __launch_bounds__(256, 3) k_conv3_wgrad_tile(
   f32x4 acc[27];
 #pragma unroll
   for (int t = 0; t < 27; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bsum = 0.f;  // channel co0+r over the lane's voxels
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int o2 = (tile % n2) << lt2, o1 = tile / n2 % n1 * 8, o0 = tile / (n1 * n2) * T0;
     __syncthreads();  // the tile before has been read
@@ -556,7 +510,9 @@ __global__ void __launch_bounds__(256, 3) k_conv3_wgrad_tile(
     for (int ks = 0; ks < WG_ROWS / 16; ks++) {
       const int row = wave * (WG_ROWS / 4) + ks * 4 + g;
       const int a0 = row >> lt2, a2 = row & (T2 - 1);
-      const bf16x8 a = as_bf16x8(gm[row * 16 + (r ^ (row & 15))]);
+      const uint4 gq = gm[row * 16 + (r ^ (row & 15))];
+      if (ci0 == 0) bsum += wg_sum(gq);
+      const bf16x8 a = as_bf16x8(gq);
 #pragma unroll
       for (int e0 = 0; e0 < 3; e0++)
 #pragma unroll
@@ -592,22 +548,107 @@ __global__ void __launch_bounds__(256, 3) k_conv3_wgrad_tile(
   for (int t = 0; t < 27; t++)
     atomicAdd(dW + (size_t)(co0 + g * 4 + wave) * 27 * Ci + (size_t)t * Ci + ci0 + r,
               red[(t * 4 + wave) * 64 + lane]);
+  if (ci0 == 0) wg_bias(bsum, red, db + co0);
 }
 
-// db[c] += sum_v gout[v][c]; 256 % C == 0.
-__global__ void __launch_bounds__(256) k_bias_grad(const bf16_t *__restrict__ gout, int C, int V,
-                                                   int vchunk, float *__restrict__ db) {
-  __shared__ float red[256];
-  const int t = threadIdx.x, c = t % C, grp = t / C, ng = 256 / C;
-  const int vbeg = blockIdx.x * vchunk, vend = min(vbeg + vchunk, V);
-  float s = 0.f;
-  for (int v = vbeg + grp; v < vend; v += ng) s += bf2f(gout[(size_t)v * C + c]);
-  red[t] = s;
-  __syncthreads();
-  if (grp == 0) {
-    for (int k = 1; k < ng; k++) s += red[k * C + c];
-    atomicAdd(db + c, s);
+// Weight and bias gradient of the one-channel stem: k_conv3_wgrad_tile with the taps as
+// the product's columns (two blocks of 16, 27 in use), each lane shifting its tap's row.
+// Every operand gathered from memory by 2-byte loads took 465 us at 256 x 256 x 16, and
+// the bias gradients of all layers another 290 us in kernels of their own.
+__global__ void __launch_bounds__(256) k_stem_wgrad(const bf16_t *__restrict__ in,
+                                                    const bf16_t *__restrict__ gout, int Co, int d0,
+                                                    int d1, int d2, int lt2, int n1, int n2,
+                                                    int ntiles, float *__restrict__ dW,
+                                                    float *__restrict__ db) {
+  extern __shared__ uint4 wg_smem[];
+  const int T2 = 1 << lt2, T0 = WG_ROWS >> lt2, W2 = T2 + 2, NR = (T0 + 2) * W2;
+  uint4 *gm = wg_smem;                // [WG_ROWS][16] gradients
+  uint4 *im = gm + WG_ROWS * 16;      // [NR] inputs
+  uint32_t *ih = (uint32_t *)(im + NR);  // [NR] the voxels before and after a row
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int co0 = blockIdx.y * 16;
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  float bsum = 0.f;
+  int trow[2], tsh[2];  // the column's tap: its row's offset and its shift along d1
+#pragma unroll
+  for (int nb = 0; nb < 2; nb++) {
+    const int t = min(nb * 16 + r, 26);
+    trow[nb] = t / 9 * W2 + t % 3;
+    tsh[nb] = t / 3 % 3;
   }
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int o2 = (tile % n2) << lt2, o1 = tile / n2 % n1 * 8, o0 = tile / (n1 * n2) * T0;
+    __syncthreads();  // the tile before has been read
+    if (tid < 2 * WG_ROWS) {
+      const int oct = tid & 1, row = tid >> 1;
+      const int q0 = o0 + (row >> lt2), q2 = o2 + (row & (T2 - 1));
+      uint4 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        v[j] = make_uint4(0, 0, 0, 0);
+        if (q0 < d0 && q2 < d2 && o1 + j < d1)
+          v[j] = *(const uint4 *)(gout + (((size_t)q0 * d1 + o1 + j) * d2 + q2) * Co + co0 + oct * 8);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        uint32_t w[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) w[j] = k == 0 ? v[j].x : k == 1 ? v[j].y : k == 2 ? v[j].z : v[j].w;
+        const int c = oct * 8 + 2 * k;
+        gm[row * 16 + (c ^ (row & 15))] = make_uint4(wg_lo(w[0], w[1]), wg_lo(w[2], w[3]),
+                                                     wg_lo(w[4], w[5]), wg_lo(w[6], w[7]));
+        gm[row * 16 + ((c + 1) ^ (row & 15))] = make_uint4(wg_hi(w[0], w[1]), wg_hi(w[2], w[3]),
+                                                           wg_hi(w[4], w[5]), wg_hi(w[6], w[7]));
+      }
+    }
+    for (int row = 255 - tid; row < NR; row += 256) {  // from the waves without gradients on
+      const int a0 = row / W2, q0 = o0 + a0 - 1, q2 = o2 + row - a0 * W2 - 1;
+      const bool ok = (unsigned)q0 < (unsigned)d0 && (unsigned)q2 < (unsigned)d2;
+      uint32_t e[10];
+#pragma unroll
+      for (int j = 0; j < 10; j++) {
+        const int q1 = o1 + j - 1;
+        e[j] = 0u;
+        if (ok && (unsigned)q1 < (unsigned)d1) e[j] = in[((size_t)q0 * d1 + q1) * d2 + q2];
+      }
+      im[row] = make_uint4(e[1] | e[2] << 16, e[3] | e[4] << 16, e[5] | e[6] << 16, e[7] | e[8] << 16);
+      ih[row] = e[0] | e[9] << 16;
+    }
+    __syncthreads();
+    for (int ks = 0; ks < WG_ROWS / 16; ks++) {
+      const int row = wave * (WG_ROWS / 4) + ks * 4 + g;
+      const int hr = (row >> lt2) * W2 + (row & (T2 - 1));
+      const uint4 gq = gm[row * 16 + (r ^ (row & 15))];
+      bsum += wg_sum(gq);
+#pragma unroll
+      for (int nb = 0; nb < 2; nb++) {
+        const uint4 m = im[hr + trow[nb]];
+        const uint32_t h = ih[hr + trow[nb]];
+        const uint32_t s1 = (m.x >> 16) | (m.y << 16), s2 = (m.y >> 16) | (m.z << 16),
+                       s3 = (m.z >> 16) | (m.w << 16);
+        uint4 b = m;
+        if (tsh[nb] == 0) b = make_uint4(wg_lo(h, m.x), s1, s2, s3);
+        if (tsh[nb] == 2) b = make_uint4(s1, s2, s3, wg_hi(m.w, h));
+        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(gq), as_bf16x8(b), acc[nb], 0, 0, 0);
+      }
+    }
+  }
+  // lane holds tap nb*16+r and rows co0+g*4+i
+  float *red = (float *)wg_smem;  // [wave][2][4][64]
+  __syncthreads();
+#pragma unroll
+  for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[((wave * 2 + nb) * 4 + i) * 64 + lane] = acc[nb][i];
+  __syncthreads();
+#pragma unroll
+  for (int nb = 0; nb < 2; nb++) {
+    float s = 0.f;
+    for (int w = 0; w < 4; w++) s += red[((w * 2 + nb) * 4 + wave) * 64 + lane];
+    if (nb * 16 + r < 27) atomicAdd(dW + (size_t)(co0 + g * 4 + wave) * 27 + nb * 16 + r, s);
+  }
+  wg_bias(bsum, red, db + co0);
 }
 
 // 2x2x2 average pool: fine dims (d0, d1, d2) -> coarse (d0/2, d1/2, d2/2); one
@@ -935,47 +976,38 @@ void launch_conv(xt_unet *u, hipStream_t st, const bf16_t *in, int Ci, const bf1
 #undef UN_LDS
     return;
   }
-  // the stem; and 16 -> 32 channels at half resolution where d2 has no factor 8
-  const int MB = 8 / NB;
-  dim3 grid((V + 64 * MB - 1) / (64 * MB), Co / (16 * NB));
-  if (NB == 1)
-    hipLaunchKernelGGL((k_conv3<false, 8, 1>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
-                       d[0], d[1], d[2], out, relu, mask);
-  else
-    hipLaunchKernelGGL((k_conv3<true, 4, 2>), grid, dim3(256), 0, st, in, Ci, W, Kpad, bias, Co,
-                       d[0], d[1], d[2], out, relu, mask);
+  // 16 -> 32 channels at half resolution where d2 has no factor 8
+  hipLaunchKernelGGL((k_conv3<4, 2>), dim3((V + 255) / 256, Co / 32), dim3(256), 0, st, in, Ci, W,
+                     Kpad, bias, Co, d[0], d[1], d[2], out, relu, mask);
 }
 
+// forward of the stem: + bias, ReLU
+void launch_stem(hipStream_t st, const bf16_t *in, const bf16_t *W, int Kpad, const float *bias,
+                 int Co, const int *d, bf16_t *out) {
+  const int TX = pow2_divisor(d[2], 32), TY = 256 / TX;
+  hipLaunchKernelGGL(k_stem, dim3((d[2] / TX) * ((d[1] + TY - 1) / TY), Co / 16,
+                                  (d[0] + STEM_SEG - 1) / STEM_SEG),
+                     dim3(512), 0, st, in, W, Kpad, bias, Co, d[0], d[1], d[2], __builtin_ctz(TX), out);
+}
+
+// dW and db of a layer with 1 (the stem) or 16 * n input channels
 void launch_wgrad(hipStream_t st, const bf16_t *in, int Ci, const bf16_t *gout, int Co,
-                  const int *d, float *dW) {
-  if (Ci % 16 == 0 && Co % 16 == 0) {
-    // rows of 8 voxels along d1 in tiles of 8 (or 4, where d2 is less) along d2; as many
-    // workgroups as run at once (3 a CU by their LDS), each over the same number of tiles
-    const int lt2 = d[2] >= 8 ? 3 : 2, T2 = 1 << lt2, T0 = WG_ROWS >> lt2;
-    const int n2 = (d[2] + T2 - 1) / T2, n1 = (d[1] + 7) / 8, n0 = (d[0] + T0 - 1) / T0;
-    const int ntiles = n0 * n1 * n2, pairs = (Ci / 16) * (Co / 16);
-    const int per = (ntiles + std::max(1, 768 / pairs) - 1) / std::max(1, 768 / pairs);
-    const size_t lds = (size_t)WG_ROWS * 16 * sizeof(uint4) +
-                       (size_t)(T0 + 2) * (T2 + 2) * 16 * (sizeof(uint4) + sizeof(uint32_t));
-    hipLaunchKernelGGL(k_conv3_wgrad_tile, dim3((ntiles + per - 1) / per, Co / 16, Ci / 16),
-                       dim3(256), lds, st, in, Ci, gout, Co, d[0], d[1], d[2], lt2, n1, n2, ntiles,
-                       dW);
-    return;
-  }
-  const int V = d[0] * d[1] * d[2];
-  const int gy = Co / 16, gz = (27 * Ci + 63) / 64;
-  int nx = std::max(1, 2048 / (gy * gz));
-  int vchunk = (V + nx - 1) / nx;
-  vchunk = std::max(128, (vchunk + 127) / 128 * 128);
-  nx = (V + vchunk - 1) / vchunk;
-  hipLaunchKernelGGL((k_conv3_wgrad<1, 4>), dim3(nx, gy, gz), dim3(256), 0, st, in, Ci, gout, Co, d[0],
-                     d[1], d[2], vchunk, dW);
-}
-
-void launch_bias_grad(hipStream_t st, const bf16_t *gout, int C, int V, float *db) {
-  const int vchunk = std::max(256, (V + 1023) / 1024);
-  hipLaunchKernelGGL(k_bias_grad, dim3((V + vchunk - 1) / vchunk), dim3(256), 0, st, gout, C, V,
-                     vchunk, db);
+                  const int *d, float *dW, float *db) {
+  // rows of 8 voxels along d1 in tiles of 8 (or 4, where d2 is less) along d2; as many
+  // workgroups as run at once (3 a CU by their LDS), each over the same number of tiles
+  const int lt2 = d[2] >= 8 ? 3 : 2, T2 = 1 << lt2, T0 = WG_ROWS >> lt2;
+  const int n2 = (d[2] + T2 - 1) / T2, n1 = (d[1] + 7) / 8, n0 = (d[0] + T0 - 1) / T0;
+  const int ntiles = n0 * n1 * n2, cb = Ci == 1 ? 1 : Ci / 16;
+  const int nx = std::max(1, 768 / (cb * (Co / 16))), per = (ntiles + nx - 1) / nx;
+  const dim3 grid((ntiles + per - 1) / per, Co / 16, cb);
+  const size_t grad = (size_t)WG_ROWS * 16 * sizeof(uint4);
+  const size_t rows = (size_t)(T0 + 2) * (T2 + 2) * (sizeof(uint4) + sizeof(uint32_t));
+  if (Ci == 1)
+    hipLaunchKernelGGL(k_stem_wgrad, grid, dim3(256), grad + rows, st, in, gout, Co, d[0], d[1], d[2],
+                       lt2, n1, n2, ntiles, dW, db);
+  else
+    hipLaunchKernelGGL(k_conv3_wgrad_tile, grid, dim3(256), grad + 16 * rows, st, in, Ci, gout, Co,
+                       d[0], d[1], d[2], lt2, n1, n2, ntiles, dW, db);
 }
 
 // forward of every layer on stream st; x is the float32 input volume
@@ -1006,7 +1038,8 @@ void enqueue_forward(xt_unet *u, const float *x, float *out, hipStream_t st) {
     hipLaunchKernelGGL(k_upcat, dim3(grid1(u->V[lvl] * (Ca + Cb) / 8)), dim3(256), 0, st, low, Ca,
                        skip, Cb, d[0], d[1], d[2], o);
   };
-  conv(0, u->t_in, u->e1a);
+  launch_stem(st, u->t_in, u->conv[0].Wf, u->conv[0].Kpad, u->params + u->conv[0].b_off, u->conv[0].Co,
+              u->dims[0], u->e1a);
   conv(1, u->e1a, u->e1);
   pool(0, u->e1, 16, u->p1);
   conv(2, u->p1, u->e2a);
@@ -1045,8 +1078,7 @@ void enqueue_backward(xt_unet *u, const float *x, const float *tgt, hipStream_t 
   auto back = [&](int l, const bf16_t *in, const bf16_t *g, bf16_t *gin, bool in_relu) {
     const Conv &c = u->conv[l];
     const int *d = u->dims[c.lvl];
-    launch_wgrad(st, in, c.Ci, g, c.Co, d, u->grads + c.w_off);
-    launch_bias_grad(st, g, c.Co, (int)u->V[c.lvl], u->grads + c.b_off);
+    launch_wgrad(st, in, c.Ci, g, c.Co, d, u->grads + c.w_off, u->grads + c.b_off);
     if (gin)
       launch_conv(u, st, g, c.Co, c.Wb, c.Kpadb, nullptr, c.Ci, d, gin, 0, in_relu ? in : nullptr);
   };
