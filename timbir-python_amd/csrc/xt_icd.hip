@@ -1083,10 +1083,15 @@ static int icd_resync(xt_icd_state *s) {
 
 template <int ZL>
 static void fbp_bp_launch(xt_icd_state *s, const float *q) {
-  constexpr int G = 256 / ZL;
-  dim3 grid((unsigned)((s->NYX + G - 1) / G), s->g.N_time);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fbp_backproject<ZL>), grid, dim3(256), 0, s->st, s->g, q,
-                     s->fbp_w, s->cosv, s->sinv, s->views, s->proj_num, s->line_mask, s->x);
+  const auto go = [&](auto k, int slices) {
+    const int G = 256 / (ZL / slices);
+    hipLaunchKernelGGL(k, dim3((unsigned)((s->NYX + G - 1) / G), s->g.N_time), dim3(256), 0, s->st, s->g,
+                       q, s->fbp_w, s->cosv, s->sinv, s->views, s->proj_num, s->line_mask, s->x);
+  };
+  if (s->g.zo == 1 && s->g.N_t == s->g.N_z && s->g.N_t % 4 == 0)  // 16-byte rows and lines
+    go(k_fbp_backproject<ZL, 4>, 4);
+  else
+    go(k_fbp_backproject<ZL, 1>, 1);
 }
 
 // Launch-shape autotuner: times one homogeneous sub-iteration (its two parity
@@ -1177,8 +1182,8 @@ static int icd_fbp(xt_icd_state *s, bool resync = true) {
   XT_TRY(dev_alloc(&q, s->nsino));
   if (s->update_offset > 0) {
     const int n = g.N_r * g.N_t;
-    hipLaunchKernelGGL(k_offset_guess_mean, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s->st,
-                       g, s->y, q);
+    hipLaunchKernelGGL(k_offset_guess_mean, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, s->st, g,
+                       s->y, q);
     hipLaunchKernelGGL(k_offset_guess_apply, dim3(1), dim3(1024), 0, s->st, g, q, s->zero_mean,
                        s->d);
   }
@@ -1187,7 +1192,9 @@ static int icd_fbp(xt_icd_state *s, bool resync = true) {
     (void)hipFree(q);
     return set_err(XT_E_ARG, "N_r=%d too large for the FBP filter", g.N_r);
   }
-  hipLaunchKernelGGL(k_fbp_filter, dim3((unsigned)((g.N_t + 3) / 4), g.N_p), dim3(256), lds, s->st,
+  // the filter's own share of that limit: rows padded by a word in 16, weights by eight
+  const size_t ns = (g.N_r + 15) / 16, flds = (4 * ns * 17 + (g.N_r + 1) / 2 + 8) * sizeof(float);
+  hipLaunchKernelGGL(k_fbp_filter, dim3((unsigned)((g.N_t + 3) / 4), g.N_p), dim3(256), flds, s->st,
                      g, s->y, s->d, q);
   switch (s->ZL) {
     case 8: fbp_bp_launch<8>(s, q); break;
