@@ -186,6 +186,16 @@ struct XtFpTable {
   const int *vpos;
 };
 
+// Workgroups of k_forward_project: an XCD takes an eighth of the views, and of those every
+// view's first chunk of bins, then every second one.  The table holds a voxel's columns
+// of consecutive views side by side (8 views in 128 bytes): the views at work together
+// read them from the XCD's L2, where one chunk after the other of a view left each XCD
+// every second view and the table was fetched eight times over (512^2 x 32 with 1024
+// views: 41 GB and 12.4 ms, now 16 GB and 10.7 ms; 256^2 x 16 in 16 frames 6.2 -> 4.9).
+inline unsigned xt_fp_grid(const XtGeom &g) {
+  return 8u * (unsigned)((g.N_p + 7) / 8) * (unsigned)((g.N_r + XT_FP_BINS - 1) / XT_FP_BINS);
+}
+
 template <int ZL, int MA, bool TAB = false>
 __global__ void __launch_bounds__(256) k_forward_project(XtGeom g, const float *__restrict__ x,
                                                          const float *__restrict__ Hr,
@@ -203,7 +213,10 @@ __global__ void __launch_bounds__(256) k_forward_project(XtGeom g, const float *
   __shared__ double acc[(XT_FP_BINS + 1) * ZL];
   __shared__ float cval[G][ZL][MA];
   __shared__ int cfirst[G][ZL];
-  const int v = blockIdx.y, j0 = blockIdx.x * XT_FP_BINS;
+  // workgroup L runs on XCD L % 8 (xt_fp_grid)
+  const int per = (g.N_p + 7) / 8, L8 = (int)(blockIdx.x >> 3);
+  const int v = (int)(blockIdx.x & 7) * per + L8 % per, j0 = L8 / per * XT_FP_BINS;
+  if (v >= g.N_p) return;
   const int tid = threadIdx.x, zl = tid % ZL, grp = tid / ZL;
   for (int q = tid; q < (XT_FP_BINS + 1) * ZL; q += 256) acc[q] = 0.0;
   __syncthreads();
