@@ -5,6 +5,7 @@ bound the difference."""
 import numpy as np
 import pytest
 
+from test_zz_no_alloc import _Hip
 from timbir_python_amd import xt_hip
 
 pytestmark = pytest.mark.gpu
@@ -14,7 +15,6 @@ pytestmark = pytest.mark.gpu
                                    (65, 257, 3), (90, 4100, 8), (40, 8192, 5)])
 @pytest.mark.parametrize("zero_mean", [True, False])
 def test_offset_split(shape, zero_mean):
-    import torch
     rng = np.random.default_rng(shape[1])
     w = rng.uniform(1e3, 1e4, shape).astype(np.float32)
     e = (rng.standard_normal(shape) / np.sqrt(w)).astype(np.float32)
@@ -26,10 +26,13 @@ def test_offset_split(shape, zero_mean):
     den = np.where(small, W, 0.4 * np.sqrt(W) / np.abs(E)).sum(0)
     gamma = (D + num / den).sum() / (1 / den).sum() if zero_mean else 0.0
     step = (num - gamma) / den
-    te, tw, td = (torch.from_numpy(a).cuda() for a in (e, w, d))
-    torch.cuda.synchronize()
-    xt_hip.offset_update_noalloc(*shape, 4.0, 0.1, zero_mean, te.data_ptr(), tw.data_ptr(),
-                                 td.data_ptr())
+    hip = _Hip()
+    try:
+        te, tw, td = (hip.upload(a) for a in (e, w, d))
+        xt_hip.offset_update_noalloc(*shape, 4.0, 0.1, zero_mean, te, tw, td)
+        eg, dg = hip.download(te, e), hip.download(td, d)
+    finally:
+        hip.free()
     ulp = np.finfo(np.float32).eps
-    assert np.abs(te.cpu().numpy() - (E - step)).max() <= 4 * ulp * np.abs(E - step).max()
-    assert np.abs(td.cpu().numpy() - (D + step)).max() <= 4 * ulp * np.abs(D + step).max()
+    assert np.abs(eg - (E - step)).max() <= 4 * ulp * np.abs(E - step).max()
+    assert np.abs(dg - (D + step)).max() <= 4 * ulp * np.abs(D + step).max()
