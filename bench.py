@@ -494,7 +494,7 @@ def main():
             conv = conv if "fbp" in conv else None
             like = (cpu_comparison(cfg, work, xt_hip) if a.workload == "slab" and not partial
                     else None)
-        # the ceiling of the line kernel's e update: its atomic write pattern alone
+        # the ceiling of an e update by memory atomics: the line kernel's write pattern alone
         atomic_rate = None
         if a.workload == "slab":
             atomic_rate = xt_hip.probe_footprint_atomics()
@@ -516,7 +516,7 @@ def main():
     # HBM bytes per launch of the voxel-update kernel measured with rocprofv3
     # FETCH_SIZE / WRITE_SIZE on this workload, scaled by a 1 GiB copy
     traffic = None
-    tf = os.path.join(ROOT, "profiles", "k_icd_lines_slab512x512x32_traffic.json")
+    tf = os.path.join(ROOT, "profiles", "k_icd_pass_slab512x512x32_traffic.json")
     if os.path.exists(tf) and a.workload == "slab":
         traffic = json.load(open(tf))["traffic_bytes_per_launch"]
     out = {
@@ -547,7 +547,8 @@ def main():
                                        "/ summed launch duration (HIP events on the library "
                                        f"stream, {KERNEL_TIMING_STEPS} iterations after the "
                                        "timed ones)",
-                     "kernel": "k_icd_lines_pc" if a.workload == "pc" else "k_icd_lines",
+                     "kernel": ("k_icd_lines_pc" if a.workload == "pc" else
+                                "k_icd_plane + k_icd_step (one launch here: a pass of both)"),
                      "kernel_ms_per_launch": g["kt_kernel_ms"] / max(1, g["kt_launches"]),
                      "bytes_per_launch": 12.0 * g["kt_footprint"] / max(1, g["kt_launches"]),
                      "launches_per_step": g["launches"] / a.steps,
@@ -563,7 +564,8 @@ def main():
                                   if g["kt_kernel_ms"] > 0 and atomic_rate else None),
                          "basis": "one FP32 atomic per footprint entry of a performed update, "
                                   "against xt_probe_footprint_atomics (the same write pattern "
-                                  "alone, same run): the line kernel's binding ceiling"}},
+                                  "alone, same run): the ceiling of a kernel that updates e "
+                                  "by memory atomics, which batched passes do not"}},
         "voxel_updates_per_step": g["updates"] / a.steps,
         "line_visits_per_step": g["visits"] / a.steps,
         "lines_in_flight_per_frame": g["lines_in_flight"],

@@ -99,7 +99,8 @@ enum {
   XT_OPT_INIT_FBP = 13,      /* 1: with initICD 0, ICD_BackProject starts from the filtered
                                 backprojection of y - d instead of zero (no counterpart in
                                 the reference; default 0) */
-  XT_OPT_AUTOTUNE = 14,      /* 1: when XT_OPT_LINES is 0, xt_icd_create times one
+  XT_OPT_AUTOTUNE = 14,      /* 1: when XT_OPT_LINES is 0 and the passes run one workgroup
+                                per line in flight, xt_icd_create times one
                                 homogeneous sub-iteration with the automatic number of lines
                                 in flight and with 1/2 and 1/4 of it, restores the state, and
                                 keeps the fastest (default 1) */
@@ -128,9 +129,9 @@ enum {
                                 sinogram once per group, are switched off (default 1) */
   XT_OPT_PASS = 20           /* how a voxel-update pass runs: 0: automatic; 1: one workgroup per
                                 line in flight; 2: in batches of the lines in flight that read
-                                the same error sinogram, streamed through LDS, wherever the
-                                A-column table and slices of one detector row allow it
-                                (default 0: batches from 16 lines in flight on) */
+                                the same error sinogram, streamed through LDS, wherever
+                                slices of one detector row and absorption footprints allow
+                                it (default 0: batches from 16 lines in flight on) */
 };
 int xt_set_option(int option, double value);
 double xt_get_option(int option);
@@ -149,7 +150,7 @@ typedef struct {
   double voxel_updates;         /* performed (not zero-skipped) voxel updates */
   double footprint_entries;     /* sum over performed updates of the sinogram
                                    footprint F_v = sum_views count * z_overlap_num */
-  double icd_kernel_ms;         /* summed duration of the voxel-update launches
+  double icd_kernel_ms;         /* summed duration of the voxel-update passes
                                    (valid when timing is on) */
   int64_t icd_launches;
   double last_cost;             /* MAP cost after the last iteration (XT_OPT_COST) */
