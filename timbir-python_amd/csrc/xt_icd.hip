@@ -687,15 +687,22 @@ static int pass_steps(const xt_icd_state *s, int mode, int sub_iter, int K, int 
   return (n + gx - 1) / gx;
 }
 
+// Lines of a step at most, in voxels across the detector: lines that share no update see
+// their common bins' error twice over, and with about 2 per voxel across the detector two
+// lines of a step meet in every bin.  512^2 with 1024 lines (2.0) and 128^2 with 201 (1.6)
+// converge as the line kernel does; 256^2 stages of three-bin voxels from a coarser
+// reconstruction diverged with 803 (3.1) and converge with 512.
+constexpr double kPassOverlap = 2.0;
+
 // Lines of a step for gx lines in flight.  A line of a step misses the changes of the
 // step's earlier lines, half of them on average, one of the line kernel's nearly all that
 // are in flight; over several frames 3/2 times the lines per step follow the line
-// kernel's iterates most closely (16 frames of 256^2 x 16 with 512 lines in flight, four
-// iterations: MAP cost 7.577e8 and ring offsets 2.2e-3 apart with 768 per step, 7.568e8
-// and 3.7e-3 with 512; two runs of the line kernel 7.576e8 and 2.1e-3), on single frames
-// the same number does.
+// kernel's iterates most closely, up to kPassOverlap (but 16).
 static int pass_lines(const xt_icd_state *s, int gx) {
-  return s->g.N_time > 1 ? std::min(1024, gx + gx / 2) : gx;
+  const XtGeom &g = s->g;
+  int n = g.N_time > 1 ? std::min(1024, gx + gx / 2) : gx;
+  const double cap = kPassOverlap * (double)g.N_r * (double)g.delta_r / (double)g.delta_xy;
+  return g_opt[XT_OPT_PASS] == 2 ? n : std::max(std::min(n, (int)cap), std::min(n, 16));
 }
 
 // Whether a pass of this mode runs in batches.  NHICD lists of the per-block rule have
