@@ -131,7 +131,8 @@ enum {
                                 line in flight; 2: in batches of the lines in flight that read
                                 the same error sinogram, streamed through LDS, wherever
                                 slices of one detector row and absorption footprints allow
-                                it (default 0: batches from 16 lines in flight on) */
+                                it (default 0: batches from 16 lines in flight on, of
+                                at most two lines per voxel across the detector) */
 };
 int xt_set_option(int option, double value);
 double xt_get_option(int option);
